@@ -1574,6 +1574,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 
+// Barrier that publishes this wave's direct global->LDS loads to the
+// workgroup.  The wait is written out: the compiler waits for such a load
+// where its own wave reads the data, which in a loop may be only after the
+// barrier, when the other waves already read.
+__device__ __forceinline__ void publish_lds_loads() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // The chunk's first 32 KiB of V rows (KV head g, pages pg_s) into v_s in
 // token order: wave instruction j moves bytes [1024 j, +1024), which lie in
 // page j / (D/32).  Every instruction is issued, so the compiler can count
@@ -4842,7 +4851,7 @@ __device__ __forceinline__ void attn_prefill_fast_body(const lgx_attn_args& a) {
     auto run = [&](int tt, lds_u16* k_s, lds_u16* v_s, lds_u16* kn, lds_u16* vn, const Pg& pgn)
                    __attribute__((always_inline)) -> Pg {
         const int t0 = tt * FPA_T;
-        __syncthreads();                          // tile tt landed (every wave waited); tile tt - 1 read
+        publish_lds_loads();                      // tile tt landed; tile tt - 1 read
         if (t0 + FPA_T > Lmax) {                  // uniform: the last tile, rows past Lmax cleared in V
             for (int p = tid; p < FPA_T * CH; p += NT)
                 if (t0 + p / CH >= Lmax) *(lds_u4*)(v_s + p * 8) = make_uint4(0u, 0u, 0u, 0u);
