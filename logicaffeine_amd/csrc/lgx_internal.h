@@ -648,8 +648,6 @@ inline lgx_status act_to_t16(lgx_ctx* c, const int8_t* xq, int m, int k, int8_t*
     return launch(c, K_ACT_T16, dim3(cdiv(slots, 256)), dim3(256), a, stream);
 }
 
-// Launch of the prefill attention over B sequences x a.qpr query rows:
-// one workgroup per (sequence, KV head, chunk of the grid, block of 4 rows).
 // Fast prefill attention (binary16 MFMA flash attention, not the canonical
 // schedule): one workgroup of gq waves per (sequence, KV head, 16 query
 // positions); writes out (binary32) and / or xq / xd (Q8_0).
@@ -662,12 +660,20 @@ inline lgx_status launch_prefill_attn_fast(lgx_ctx* c, const lgx_attn_args& a, i
     if (wgs == 0) return LGX_OK;
     return launch(c, (Kern)k, dim3((unsigned)wgs), dim3(64 * gq), a, stream);
 }
+// Launch of the prefill attention over B sequences x a.qpr query rows: one
+// workgroup per (sequence, KV head, chunk of the grid, block of 32 / heads
+// query rows).
 inline lgx_status launch_prefill_attn(lgx_ctx* c, const lgx_attn_args& a, int d, void* stream) {
     const int k = prefill_attn_kernel(d, a.hq / a.hkv);
-    const int64_t wgs = (int64_t)a.B * a.hkv * a.ncg * ((std::max(a.qpr, 1) + 3) / 4);
-    if (k < 0 || wgs > INT32_MAX) return fail(LGX_UNSUPPORTED, "prefill attention shape");
+    if (k < 0) return fail(LGX_UNSUPPORTED, "prefill attention shape");
+    const int qb = 32 / (a.hq / a.hkv);           // query rows per workgroup (PFA_R / heads)
+    // per chunk, the runs of LGX_PFA_SEG query blocks in eights (one per XCD)
+    const int64_t nqb = (std::max(a.qpr, 1) + qb - 1) / qb;
+    const int64_t runs = (int64_t)a.B * a.hkv * ((nqb + LGX_PFA_SEG - 1) / LGX_PFA_SEG);
+    const int64_t wgs = (runs + 7) / 8 * 8 * LGX_PFA_SEG * a.ncg;
+    if (wgs > INT32_MAX) return fail(LGX_UNSUPPORTED, "prefill attention shape");
     if (wgs == 0) return LGX_OK;
-    return launch(c, (Kern)k, dim3((unsigned)wgs), dim3(512), a, stream);
+    return launch(c, (Kern)k, dim3((unsigned)wgs), dim3(256), a, stream);
 }
 
 }  // namespace lgxi

@@ -119,6 +119,7 @@ typedef struct {
 
 #define LGX_PAGE 16
 #define LGX_ATTN_CHUNK 256
+#define LGX_PFA_SEG 4          // prefill attention: query blocks of a chunk that stay on one XCD
 
 // ---- decode-step glue ----
 typedef struct {

@@ -4425,265 +4425,336 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // max, lgx_expf, the halving-tree sum over 256 slots, the PV chain over the
 // chunk's tokens; chunks merged by attn_merge), so a prefilled position has
 // the bits of a decoded one.
-// Workgroup: 512 threads = 8 waves for (sequence b, KV head g, block of
-// PFA_QB query rows, chunk c).  The chunk's K rows, then its V rows, pass
-// through one 32 KiB LDS tile in stages of PFA_TOK tokens (direct
-// global->LDS loads; each row's 16-byte pieces are stored XOR-swizzled by
-// the row, so row-wise and column-wise reads are conflict-free) and serve
-// the PFA_QB rows x GQ heads.
-//   scores:  wave (row qp = w/2, head group hg = w%2) owns heads
-//            4 hg .. 4 hg + 3 over the whole chunk, lane l the tokens
-//            l + 64 u; the query values come through the scalar cache
-//            (uniform in the wave), 4 heads x 8 dimensions per step.
-//   softmax: within the wave: per head the max, p to LDS, the halving tree
+// The two chains run on the binary32 matrix instructions: each accumulates
+// its K products one after the other with a rounding per step, i.e. it is
+// the fmaf chain of the schedule (checked bit for bit over normal, subnormal,
+// infinite and NaN operands).  A step costs the same cycles as the VALU's
+// fmaf of 64 lanes but takes 32 rows against one converted K or V value, so
+// the conversions, the LDS reads and the query broadcasts are shared by all
+// rows.
+// Workgroup: 4 waves for (sequence b, KV head g, PFA_QB query rows, chunk c);
+// the (query row, head) pairs of the group, row-major, are the PFA_R = 32
+// rows of the products.
+//   scores:  wave w owns tokens 64 w + lane (the lane's K row in registers);
+//            v_mfma_f32_32x32x1 (two blocks of 32 tokens), the query rows
+//            from LDS as the A operand, block 0's values of the even and odd
+//            halves of 8 dimensions broadcast to both blocks in turn.
+//   softmax: the raw scores go through LDS; wave w takes rows 8 w ..: lane l
+//            the tokens l + 64 u, the max, p back to LDS, the halving tree
 //            (levels 128 and 64 in-lane, the rest across lanes).
-//   PV:      wave (row qp = w/2, head group w%2); 16-lane row rho is head
-//            4 (w%2) + rho, lane k owns dims [D/16 k, +D/16); the row's p_t
-//            comes from lane t%16 of a 16-token register (DPP row_newbcast).
+//   PV:      wave w owns dimensions [w D/4, +D/4) of all rows;
+//            v_mfma_f32_16x16x4, A = p (a lane's tokens 16 u + 4 e + g are
+//            neighbours in LDS: pfa_pos), B = V through the transposing LDS
+//            load.  V passes through two 8 KiB buffers by direct
+//            global->LDS loads, 16-byte pieces swizzled by the row.
+// 50 KiB of LDS and at most 168 VGPRs: three workgroups per compute unit,
+// whose softmax and loads overlap the others' matrix work.
+// Bound by the binary32 matrix rate (65 cycles for 2048 products; 140 us of
+// it below).  8 sequences x 128 rows at contexts up to 2000, 28/4 heads of
+// 128: 253 us, against 641 us with the chains on the VALU (8 waves, four
+// query rows, query values through scalar registers) and 387 us with each
+// XCD given whole sequences, whose lengths differ.
+// Rows of a block end at different tokens: p is 0 past a row's length, which
+// leaves o as it is unless V there is infinite or NaN; the last groups of 16
+// tokens (those that some row does not attend to in full) clear V past the
+// block's last length and, if they hold a V value that is not finite, run
+// the chain on the VALU row by row.  (o is never -0: p is 0 or above 2^-126,
+// so no product underflows to 0.)
 // ---------------------------------------------------------------------------
-#define PFA_QB 4
+#define PFA_R 32
+#define PFA_SEG LGX_PFA_SEG
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
+
+// lgx_expf for x <= 0 or NaN: the same operations without the branches that
+// such an x cannot take; the exponent field comes from the low bits of the
+// rounded sum 1.5 * 2^23 + n.
+__device__ __forceinline__ float lgx_expf_nonpos(float x) {
+    const float t = x * 1.44269504088896341f;
+    const float u = t + 12582912.0f;
+    const float nf = u - 12582912.0f;
+    float r = fmaf(-nf, 0.693145751953125f, x);
+    r = fmaf(-nf, 1.42860682030941723e-06f, r);
+    float p = 1.98412698412698413e-04f;
+    p = fmaf(p, r, 1.38888888888888889e-03f);
+    p = fmaf(p, r, 8.33333333333333333e-03f);
+    p = fmaf(p, r, 4.16666666666666667e-02f);
+    p = fmaf(p, r, 1.66666666666666667e-01f);
+    p = fmaf(p, r, 0.5f);
+    p = fmaf(p, r, 1.0f);
+    p = fmaf(p, r, 1.0f);
+    const float e = p * __uint_as_float((__float_as_uint(u) << 23) + 0x3f800000u);
+    return x < -87.33f ? 0.0f : e;
+}
+
+// Column of token t in a p row: the tokens 16 u + 4 e + g, e = 0..3, of one
+// PV operand lane group g side by side.
+__device__ __forceinline__ int pfa_pos(int t) { return (t & ~15) + 4 * (t & 3) + ((t >> 2) & 3); }
+
+// Swizzle of the 16-byte pieces of V row t in LDS: 32-byte pairs spread so
+// that the 16 rows of a transposing load fall on different pairs.
 template <int D>
 __device__ __forceinline__ int pfa_swz(int t) {
-    return D == 128 ? (t & 15) : ((t >> 1) & 7);
+    return D == 128 ? (t & 7) << 1 : ((t >> 1) & 3) << 1;
 }
 
 template <int D, int GQ>
 __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     constexpr int C = LGX_ATTN_CHUNK;
-    constexpr int TOK = 32768 / (2 * D);          // tokens per K/V stage
-    constexpr int NST = C / TOK;
+    constexpr int QB = PFA_R / GQ;                // query rows of the workgroup
     constexpr int CPR = D / 8;                    // 16-byte pieces per row
-    constexpr int NU = TOK / 128;                 // tokens per lane per stage
-    __shared__ __align__(16) uint16_t kv_s[TOK * D];
-    // p rows padded by 16 floats: the four heads of a wave read the same
-    // token column in four distinct bank groups
-    __shared__ __align__(16) float p_s[PFA_QB][GQ][C + 16];
+    constexpr int QS = D + 4, PS = C + 8;         // row strides in floats
+    constexpr int VT = 8192 / (2 * D);            // tokens per V buffer
+    constexpr int NC = D / 64;                    // 16-dimension column tiles per wave
+    // the query rows, then (once every wave has its scores) the p rows
+    __shared__ __align__(16) float p_s[PFA_R * PS];
+    // two buffers as two variables: a direct load into one is known not to
+    // alias reads of the other
+    __shared__ __align__(16) uint16_t vb0[VT * D], vb1[VT * D];
     __shared__ int pg_s[C / LGX_PAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qpr = max(a.qpr, 1);
-    const int nqb = (qpr + PFA_QB - 1) / PFA_QB;
-    // XCD-aware logical id, then (sequence x KV head, chunk, query block):
-    // the blocks that share a chunk's K/V run on one XCD together
-    const int T = a.B * a.hkv * a.ncg * nqb;
-    const int P = blockIdx.x, xcd = P & 7, slot = P >> 3;
-    const int id = xcd * (T >> 3) + min(xcd, T & 7) + slot;
-    const int bg = id / (a.ncg * nqb), rem = id - bg * (a.ncg * nqb);
-    const int c = rem / nqb, qb = rem - c * nqb;
+    const int nqb = (qpr + QB - 1) / QB;
+    // physical ids go round-robin over the 8 XCDs.  A run of PFA_SEG query
+    // blocks of one (chunk, sequence x KV head) stays on one XCD, whose L2
+    // serves their K/V; the runs of a chunk index go round the XCDs, one step
+    // further with each chunk, so that sequences of different lengths (whose
+    // later chunks are empty) load all XCDs alike
+    const int nseg = (nqb + PFA_SEG - 1) / PFA_SEG;
+    const int nrun = a.B * a.hkv * nseg, nrun8 = (nrun + 7) >> 3;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int ri = slot / PFA_SEG;
+    const int c = ri / nrun8;
+    const int run = 8 * (ri - c * nrun8) + ((xcd - c) & 7);
+    if (run >= nrun) return;
+    const int bg = run / nseg, qb = (run - bg * nseg) * PFA_SEG + slot % PFA_SEG;
+    if (qb >= nqb) return;
     const int b = bg / a.hkv, g = bg - b * a.hkv;
-    const int j0 = qb * PFA_QB, t0 = c * C;
+    const int j0 = qb * QB, t0 = c * C;
     const int sl = a.seq_len[b];
-    const int jl = min(j0 + PFA_QB, qpr) - 1;              // last row of the block
-    const int Lmax = min(max(sl + jl + a.len_add, 0), a.maxlen);
-    if (t0 >= Lmax) return;                       // whole workgroup, before any barrier
+    // tokens of this chunk that query row j of the sequence attends to
+    auto n_of = [&](int j) { return min(C, min(max(sl + j + a.len_add, 0), a.maxlen) - t0); };
+    const int nmax = n_of(min(j0 + QB, qpr) - 1);          // the block's last row
+    if (nmax <= 0) return;                        // whole workgroup, before any barrier
+    const int nmin = max(n_of(j0), 0);
     if (tid < C / LGX_PAGE) {
         int pg = 0;
-        if (t0 + tid * LGX_PAGE < Lmax) pg = a.page_table[(int64_t)b * a.maxp + t0 / LGX_PAGE + tid];
+        if (tid * LGX_PAGE < nmax) pg = a.page_table[(int64_t)b * a.maxp + t0 / LGX_PAGE + tid];
         pg_s[tid] = min(max(pg, 0), a.num_pages - 1);
+    }
+    // query rows: row r is (query row r / GQ, head r % GQ); rows past the
+    // last one repeat it and are never written out
+    for (int i = tid; i < PFA_R * D / 4; i += 256) {
+        const int r = min(i / (D / 4), QB * GQ - 1), col = (i % (D / 4)) * 4;
+        const int jr = min(j0 + r / GQ, qpr - 1);
+        *(float4*)(p_s + (i / (D / 4)) * QS + col) =
+            *(const float4*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + col);
     }
     __syncthreads();
 
-    // direct loads of stage kap (tokens [kap TOK, +TOK) of the chunk) of K
-    // or V: 32 wave instructions of 1 KiB, wave w issues w, w + 8, ...
-    auto stage = [&](const uint16_t* pages, int kap) {
+    // direct loads of V tokens [VT k, +VT) of the chunk: 8 wave instructions
+    // of 1 KiB
+    auto stage_v = [&](uint16_t* vb, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < TOK * CPR / 64 / 8; ++i) {
-            const int ins = wave + 8 * i;
-            const int pos = ins * 64 + lane;
-            const int t = pos / CPR, sp = pos - t * CPR;
-            const int tok = kap * TOK + t;
-            const uint16_t* src = pages +
+        for (int i = 0; i < 2; ++i) {
+            const int ins = wave + 4 * i;
+            const int t = ins * (64 / CPR) + lane / CPR, sp = lane % CPR;
+            const int tok = k * VT + t;
+            const uint16_t* src = a.vpages +
                 (((int64_t)pg_s[tok >> 4] * a.hkv + g) * LGX_PAGE + (tok & 15)) * D + (sp ^ pfa_swz<D>(t)) * 8;
-            __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(kv_s + ins * 512), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(vb + ins * 512), 16, 0, 0);
         }
     };
 
-    // ---- scores: wave (row qp, head group hg) owns heads 4 hg + hh (hh < 4)
-    // over all C tokens of the chunk, lane l the tokens l + 64 u (u < 4) ----
-    constexpr int HW = 4;                         // heads per wave
-    constexpr int UPS = TOK / 64;                 // tokens per lane per stage
-    const int qp = wave >> 1, hg = wave & 1;
-    const int jq = j0 + qp;
-    const int row = b * qpr + min(jq, qpr - 1);
-    const int nq = jq < qpr ? min(C, min(max(sl + jq + a.len_add, 0), a.maxlen) - t0) : 0;
-    typedef const __attribute__((address_space(4))) float* qptr_t;
-    const qptr_t q0 = (qptr_t)(a.q + ((int64_t)row * a.hq + g * GQ) * D);
-    int qoff[HW];                                 // heads past GQ re-read the last one
+    // ---- scores ----
+    v32f s = {};
+    {
+        const int tok = 64 * wave + lane;
+        const uint4* kr = (const uint4*)(a.kpages +
+            (((int64_t)pg_s[tok >> 4] * a.hkv + g) * LGX_PAGE + (tok & 15)) * D);
+        uint4 kv[CPR];
 #pragma unroll
-    for (int hh = 0; hh < HW; ++hh) qoff[hh] = min(4 * hg + hh, GQ - 1) * D;
-    auto qh_at = [&](int hh, int i) { return q0[qoff[hh] + i]; };
-    float sc[HW][4];
+        for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
+        // K lands before V is requested (the compiler waits for every load in
+        // flight once direct loads are among them); V arrives meanwhile
 #pragma unroll
-    for (int kap = 0; kap < NST; ++kap) {
-        if (kap > 0) __syncthreads();             // the previous stage is fully read
-        stage(a.kpages, kap);
-        __syncthreads();                          // every wave's loads have landed
-        float acc[HW][UPS];
+        for (int j = 0; j < CPR; ++j)
+            asm volatile("" : "+v"(kv[j].x), "+v"(kv[j].y), "+v"(kv[j].z), "+v"(kv[j].w));
+        stage_v(vb0, 0);
+        const float* qr = p_s + (lane & 31) * QS + 4 * (lane >> 5);
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh)
-#pragma unroll
-            for (int v = 0; v < UPS; ++v) acc[hh][v] = 0.0f;
-        // 8 dimensions per step (one 16-byte K read per token), the query
-        // values in two halves of 4 x 4 scalar registers: each half is
-        // requested one half-step before its products
-        float qa[HW][4], qb[HW][4];
-        auto qload = [&](float (&qv)[HW][4], int s4) {
-#pragma unroll
-            for (int hh = 0; hh < HW; ++hh)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) qv[hh][e] = qh_at(hh, 4 * s4 + e);
-        };
-        auto qk_half = [&](const float (&qv)[HW][4], const float (&kf)[UPS][8], int e0) {
+        for (int j = 0; j < CPR; ++j) {
+            const float4 q4 = *(const float4*)(qr + 8 * j);
+            const uint32_t w4[4] = {kv[j].x, kv[j].y, kv[j].z, kv[j].w};
+            const float qa[4] = {q4.x, q4.y, q4.z, q4.w};
 #pragma unroll
             for (int e = 0; e < 4; ++e)
+                s = __builtin_amdgcn_mfma_f32_32x32x1f32(
+                    qa[e], h2f(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu), s, 1, 0, 0);
 #pragma unroll
-                for (int hh = 0; hh < HW; ++hh)
-#pragma unroll
-                    for (int v = 0; v < UPS; ++v)
-                        acc[hh][v] = fmaf(qv[hh][e], kf[v][e0 + e], acc[hh][v]);
-        };
-        qload(qa, 0);
-#pragma unroll 1
-        for (int s8 = 0; s8 < CPR; ++s8) {
-            float kf[UPS][8];
-#pragma unroll
-            for (int v = 0; v < UPS; ++v) {
-                const int t = lane + 64 * v;
-                const uint4 kv = *(const uint4*)(kv_s + t * D + (s8 ^ pfa_swz<D>(t)) * 8);
-                const uint32_t w4[4] = {kv.x, kv.y, kv.z, kv.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    kf[v][2 * e] = h2f(w4[e] & 0xffffu);
-                    kf[v][2 * e + 1] = h2f(w4[e] >> 16);
-                }
-            }
-            qload(qb, 2 * s8 + 1);
-            qk_half(qa, kf, 0);
-            if (s8 + 1 < CPR) qload(qa, 2 * s8 + 2);
-            qk_half(qb, kf, 4);
+            for (int e = 0; e < 4; ++e)
+                s = __builtin_amdgcn_mfma_f32_32x32x1f32(
+                    qa[e], h2f(e & 1 ? w4[2 + (e >> 1)] >> 16 : w4[2 + (e >> 1)] & 0xffffu), s, 1, 1, 0);
         }
-#pragma unroll
-        for (int hh = 0; hh < HW; ++hh)
-#pragma unroll
-            for (int v = 0; v < UPS; ++v) sc[hh][kap * UPS + v] = acc[hh][v] * a.scale;
     }
-    __syncthreads();                              // K fully read: the tile takes V
-    stage(a.vpages, 0);
-
-    // ---- softmax, within the wave: max, p to LDS, halving tree (levels
-    // 128 and 64 in-lane, the rest across lanes); the wave's heads advance
-    // each shuffle level together ----
-    {
-        float mm[HW], l[HW];
+    // lane l holds, of token 64 w + 32 blk + l % 32, the rows
+    // 8 (i / 4) + 4 (l / 32) + i % 4
+    __syncthreads();                              // the query rows are fully read
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) {
-            mm[hh] = -__builtin_inff();
+    for (int blk = 0; blk < 2; ++blk) {
+        float* pc = p_s + 4 * (lane >> 5) * PS + pfa_pos(64 * wave + 32 * blk + (lane & 31));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pc[(8 * (i >> 2) + (i & 3)) * PS] = s[16 * blk + i];
+    }
+    __syncthreads();
+
+    // ---- softmax of rows 8 w .. 8 w + 7, four at a time ----
+#pragma unroll
+    for (int rb = 0; rb < 8; rb += 4) {
+        float p[4][4], mm[4], l[4];
+        int nr[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 8 * wave + rb + i, jr = j0 + r / GQ;
+            nr[i] = r < QB * GQ && jr < qpr ? n_of(jr) : 0;
+            mm[i] = -__builtin_inff();
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                sc[hh][u] = lane + 64 * u < nq ? sc[hh][u] : -__builtin_inff();
-                mm[hh] = fmaxf(mm[hh], sc[hh][u]);
+                p[i][u] = lane + 64 * u < nr[i] ? p_s[r * PS + pfa_pos(lane + 64 * u)] * a.scale : -__builtin_inff();
+                mm[i] = fmaxf(mm[i], p[i][u]);
             }
         }
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) mm[hh] = wave_max(mm[hh]);
+        for (int i = 0; i < 4; ++i) mm[i] = wave_max(mm[i]);
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) {
-            const int h = 4 * hg + hh;
-            float p[4];
+        for (int i = 0; i < 4; ++i) {
+            const int r = 8 * wave + rb + i;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) p[u] = lane + 64 * u < nq ? lgx_expf(sc[hh][u] - mm[hh]) : 0.0f;
-            if (h < GQ) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) p_s[qp][h][lane + 64 * u] = p[u];
+            for (int u = 0; u < 4; ++u) {
+                p[i][u] = lane + 64 * u < nr[i] ? lgx_expf_nonpos(p[i][u] - mm[i]) : 0.0f;
+                p_s[r * PS + pfa_pos(lane + 64 * u)] = p[i][u];
             }
-            l[hh] = (p[0] + p[2]) + (p[1] + p[3]);  // levels 128 and 64
+            l[i] = (p[i][0] + p[i][2]) + (p[i][1] + p[i][3]);   // levels 128 and 64
         }
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) l[hh] = wave_tree_sum(l[hh]);
-        if (lane == 0 && nq > 0) {
+        for (int i = 0; i < 4; ++i) l[i] = wave_tree_sum(l[i]);
+        if (lane == 0) {
 #pragma unroll
-            for (int hh = 0; hh < HW; ++hh) {
-                const int h = 4 * hg + hh;
-                if (h < GQ) {
-                    float* pp = a.part + (((int64_t)row * a.hq + g * GQ + h) * a.nchunk + c) * (D + 2);
-                    pp[D] = mm[hh];
-                    pp[D + 1] = l[hh];
+            for (int i = 0; i < 4; ++i) {
+                const int r = 8 * wave + rb + i;
+                if (nr[i] > 0) {
+                    float* pp = a.part + ((((int64_t)b * qpr + j0 + r / GQ) * a.hq + g * GQ + r % GQ) * a.nchunk + c) * (D + 2);
+                    pp[D] = mm[i];
+                    pp[D + 1] = l[i];
                 }
             }
         }
     }
 
     // ---- PV ----
-    constexpr int DL = D / 16;
-    const int rho = lane >> 4, k = lane & 15;
-    const int h = 4 * hg + rho, hc = min(h, GQ - 1);
-    float o[DL];
+    const int qc = lane & 15, kg = lane >> 4;
+    v4f o[2][NC];
 #pragma unroll
-    for (int e = 0; e < DL; ++e) o[e] = 0.0f;
-    // a lane's DL halves of V row t of the stage tile (uint4: DL = 8; .xy: DL = 4)
-    auto v_load = [&](int t) -> uint4 {
-        const int sw = pfa_swz<D>(t);
-        if constexpr (D == 128) {
-            return *(const uint4*)(kv_s + t * D + (k ^ sw) * 8);
-        } else {
-            const uint2 vv = *(const uint2*)(kv_s + t * D + ((k >> 1) ^ sw) * 8 + (k & 1) * 4);
-            return make_uint4(vv.x, vv.y, 0u, 0u);
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) o[rt][ct] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    auto pv_load = [&](uint16_t* vb, int ts, int k, float4 (&pa)[2], float (&vf)[NC][4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) pa[rt] = *(const float4*)(p_s + (16 * rt + qc) * PS + ts + 4 * kg);
+        // lane (qc, kg) loads token ts + 4 (qc / 4) + kg, dimensions
+        // 4 (qc % 4) .. of the column tile, and receives dimension qc of the
+        // tokens ts + 4 e + kg
+        const int tv = ts - k * VT + 4 * (qc >> 2) + kg;
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) {
+            const int cv = 2 * (wave * NC + ct) + ((qc >> 1) & 1);
+            const v4s vw = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_v4s*)(vb + tv * D + (cv ^ pfa_swz<D>(tv)) * 8 + (qc & 1) * 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vf[ct][e] = h2f((uint16_t)vw[e]);
         }
     };
-    auto pv_apply = [&](const uint4 vv, float pb) {
-        const uint32_t w4[4] = {vv.x, vv.y, vv.z, vv.w};
-        float vf[8];
+    auto pv_mul = [&](const float4 (&pa)[2], const float (&vf)[NC][4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            vf[2 * e] = h2f(w4[e] & 0xffffu);
-            vf[2 * e + 1] = h2f(w4[e] >> 16);
-        }
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int e = 0; e < DL; ++e) o[e] = fmaf(pb, vf[e], o[e]);
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) {
+                    const float pe = e == 0 ? pa[rt].x : e == 1 ? pa[rt].y : e == 2 ? pa[rt].z : pa[rt].w;
+                    o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(pe, vf[ct][e], o[rt][ct], 0, 0, 0);
+                }
     };
-#pragma unroll
-    for (int kap = 0; kap < NST; ++kap) {
-        if (kap > 0) {
-            __syncthreads();
-            stage(a.vpages, kap);
+    auto pv_stage = [&](uint16_t* vb, uint16_t* vn, int k) __attribute__((always_inline)) {
+        publish_lds_loads();                      // stage k landed; stage k - 1 fully read; p written
+        if ((k + 1) * VT < nmax) stage_v(vn, k + 1);
+        const int te = min(nmax, (k + 1) * VT);
+        const int tf = min(te, nmin) & ~15;       // groups before it: every row attends in full
+        int ts = k * VT;
+        for (; ts < tf; ts += 16) {
+            float4 pa[2];
+            float vf[NC][4];
+            pv_load(vb, ts, k, pa, vf);
+            pv_mul(pa, vf);
         }
-        __syncthreads();                          // V stage kap has landed
-        const int tb = kap * TOK, te = min(nq, tb + TOK);   // uniform in the wave
-        for (int ts = tb; ts < te; ts += 16) {
-            // p of the 16 tokens: four 16-byte reads at one address per
-            // 16-lane row (LDS broadcast)
-            float pt[16];
-            static_for<0, 4>([&](auto Q) {
-                const float4 p4 = *(const float4*)&p_s[qp][hc][ts + 4 * Q.value];
-                pt[4 * Q.value] = p4.x;
-                pt[4 * Q.value + 1] = p4.y;
-                pt[4 * Q.value + 2] = p4.z;
-                pt[4 * Q.value + 3] = p4.w;
-            });
-            if (ts + 16 <= te) {
-                // 8 rows' reads issued together, then their chains (twice)
-                uint4 va[8];
-                static_for<0, 8>([&](auto J) { va[J.value] = v_load(ts + J.value - tb); });
-                static_for<0, 8>([&](auto J) { pv_apply(va[J.value], pt[J.value]); });
-                static_for<0, 8>([&](auto J) { va[J.value] = v_load(ts + 8 + J.value - tb); });
-                static_for<0, 8>([&](auto J) { pv_apply(va[J.value], pt[8 + J.value]); });
-            } else {
-                static_for<0, 16>([&](auto J) {
-                    if (ts + J.value < te) pv_apply(v_load(ts + J.value - tb), pt[J.value]);
-                });
+        for (; ts < te; ts += 16) {               // a row ends in here
+            float4 pa[2];
+            float vf[NC][4];
+            pv_load(vb, ts, k, pa, vf);
+            bool bad = false;
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (ts + 4 * e + kg >= nmax) vf[ct][e] = 0.0f;
+                    bad |= !(fabsf(vf[ct][e]) < __builtin_inff());
+                }
+            if (__builtin_amdgcn_ballot_w64(bad) == 0) {
+                pv_mul(pa, vf);
+                continue;
+            }
+            for (int t = ts; t < min(ts + 16, nmax); ++t) {
+                const int tr = t - k * VT;
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    const int col = 16 * (wave * NC + ct) + qc;
+                    const float v = h2f(vb[tr * D + ((col >> 3) ^ pfa_swz<D>(tr)) * 8 + (col & 7)]);
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int r = 16 * rt + 4 * kg + i;
+                            if (t < n_of(j0 + r / GQ))
+                                o[rt][ct][i] = fmaf(p_s[r * PS + pfa_pos(t)], v, o[rt][ct][i]);
+                        }
+                }
             }
         }
+    };
+#pragma unroll 1
+    for (int k = 0; k * VT < nmax; k += 2) {
+        pv_stage(vb0, vb1, k);
+        if ((k + 1) * VT < nmax) pv_stage(vb1, vb0, k + 1);
     }
-    if (h < GQ && nq > 0) {
-        float* pp = a.part + (((int64_t)row * a.hq + g * GQ + h) * a.nchunk + c) * (D + 2) + DL * k;
 #pragma unroll
-        for (int e = 0; e < DL; e += 4) *(float4*)(pp + e) = make_float4(o[e], o[e + 1], o[e + 2], o[e + 3]);
-    }
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * rt + 4 * kg + i, jr = j0 + r / GQ;
+            if (r >= QB * GQ || jr >= qpr || n_of(jr) <= 0) continue;
+            float* pp = a.part + ((((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * a.nchunk + c) * (D + 2) +
+                        16 * wave * NC + qc;
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) pp[16 * ct] = o[rt][ct][i];
+        }
 }
 
 #define LGX_PFA_KERNELS(D, G)                                                                     \
-    extern "C" __global__ __launch_bounds__(512) void lgx_k_attn_prefill_d##D##_g##G(            \
-        const lgx_attn_args a) {                                                                 \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))        \
+    void lgx_k_attn_prefill_d##D##_g##G(const lgx_attn_args a) {                                                                 \
         attn_prefill_body<D, G>(a);                                                              \
     }
 LGX_PFA_KERNELS(64, 1)
@@ -4728,8 +4799,6 @@ LGX_PFA_KERNELS(128, 8)
 // ---------------------------------------------------------------------------
 #define FPA_Q 16
 #define FPA_T 64
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4s lds_v4s;
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef __attribute__((address_space(3))) uint4 lds_u4;
 // Tile staging: direct global->LDS loads into two buffers, the next tile's

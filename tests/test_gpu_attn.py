@@ -171,6 +171,29 @@ def test_prefill_attn_head_groups_bit_exact(ctx, orc, g, d):
     assert np.array_equal(out, prefill_ref(orc, q, k, v, pt, ctx_len, P))
 
 
+@pytest.mark.parametrize("hq,hkv,d,P", [(14, 2, 64, 21), (28, 4, 128, 5), (2, 2, 128, 33), (9, 3, 64, 1)])
+def test_prefill_attn_values_some_rows_do_not_attend_to(ctx, orc, hq, hkv, d, P):
+    """Infinite and NaN V rows inside the last rows' reach: rows before them
+    keep their finite bits, rows from them on get the oracle's infinities and
+    NaN (the 0 weight of a row that ends earlier must not meet such a value).
+    One, two and three blocks of query rows, one with a cut at max_seq_len."""
+    ctx_len = [0, 250, 37]
+    B = len(ctx_len)
+    k, v, pt, maxp = make_cache(B, hkv, d, [c + P for c in ctx_len], seed=3 * d + P)
+    for b, c in enumerate(ctx_len):
+        for pos, val in ((c + P // 2, np.inf), (c + P - 1, np.nan)):
+            v[pt[b, pos // 16], :, pos % 16, 3::7] = np.float16(val).view(np.uint16)
+    q = orc.gen_normal_f32(6, d + P, (B * P, hq, d))
+    msl = 250 + P - 1 if P > 1 else 251        # the second sequence's last row is clamped
+    out = host(ctx.gqa_prefill_attn(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v),
+                                    ctx.to_device(pt), ctx.to_device(np.asarray(ctx_len, np.int32)),
+                                    P, msl))
+    lens = np.minimum([c + j + 1 for c in ctx_len for j in range(P)], msl).astype(np.int32)
+    ref = orc.gqa_decode_attn(q, k, v, np.repeat(pt, P, axis=0), lens)
+    assert np.isfinite(ref).any() and not np.isfinite(ref).all()
+    assert np.array_equal(out, ref, equal_nan=True)
+
+
 def test_prefill_attn_config4_shape_sampled(ctx, orc):
     """Config-4 head layout at a 4096-token context: 64 new rows after 4032
     cached tokens (17 chunks), checked on a sample of rows."""
