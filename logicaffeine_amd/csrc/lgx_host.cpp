@@ -515,7 +515,7 @@ static lgx_status q8_gemm_impl(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
     if (m >= c->tiled_min) {
         // T16 copy of the activations, then the group partials (straight
         // into y when K is one group) and the tree over the groups
-        const Kern kern = tiled_kernel(c, m);
+        const Kern kern = tiled_kernel(c, W->n, W->k, m);
         const int grp = tiled_grp(c, kern, W->n, W->k, m);
         const int ng = tiled_groups(W->k, grp);
         const size_t xbytes = ((size_t)cdiv(m, 16) * 16 * W->k + 255) / 256 * 256;
@@ -578,8 +578,12 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
         // the tiled product from 17 rows (config 1 at M = 32: 28.9 us against
         // 35.4 us per step on the 16-row streaming kernels)
         const bool tiled = m >= std::min(c->tiled_min, 17);
-        const Kern tk = tiled_kernel(c, m);
-        const int trows = tk == K_GEMM_TILED ? 128 : tk == K_GEMM_TILED64 ? 64 : 32;
+        // 64-row tiles where they are worth it for the grid of all matrices
+        int64_t wgs64 = 0;
+        for (int i = 0; i < count; ++i) wgs64 += tiled64_wgs(W[i].n, W[i].k, m);
+        const Kern tk = c->tiled_rows ? tiled_kernel(c, W[0].n, W[0].k, m)
+                        : m >= 256 && wgs64 >= 600 ? K_GEMM_TILED64 : K_GEMM_TILED32;
+        const int trows = tiled_rows_of(tk);
         // ranges per group of the tiled products: 2, or 1 when that leaves
         // fewer than two workgroups per compute unit over all the matrices
         // together.  Groups of 4 make the long-K matrix's workgroups the
@@ -661,14 +665,11 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
                 a.ngroups = tiled_groups(W[i].k, grp);
                 a.ntn = (int)cdiv(W[i].n, LGX_TG_N);
                 a.ntm = (int)cdiv(m, trows);
-                const int64_t wgs = (int64_t)a.ntn * a.ntm * a.ngroups;
-                const int64_t end = ta.wg0[i] + (wgs + 7) / 8 * 8;
+                const int64_t end = ta.wg0[i] + tiled_grid(a);
                 if (end > INT32_MAX) return fail(LGX_OUT_OF_BOUNDS, "grouped product too large");
                 ta.wg0[i + 1] = (int32_t)end;
             }
-            const Kern gk = tk == K_GEMM_TILED   ? K_GEMM_TILED_GROUP
-                            : tk == K_GEMM_TILED64 ? K_GEMM_TILED64_GROUP
-                                                   : K_GEMM_TILED32_GROUP;
+            const Kern gk = tk == K_GEMM_TILED64 ? K_GEMM_TILED64_GROUP : K_GEMM_TILED32_GROUP;
             if ((st = launch(c, gk, dim3(ta.wg0[count]), dim3(256), ta, stream)) != LGX_OK) return st;
         } else {
             // 16-row m-groups (several workgroups per weight tile, the

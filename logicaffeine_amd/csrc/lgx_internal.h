@@ -138,7 +138,6 @@ enum Kern {
     K_NORM4_R8,
     K_NORM4_R20,
     K_ACT_T16,
-    K_GEMM_TILED,
     K_GEMM_TILED64,
     K_GEMM_TILED32,
     K_PFA_D64_G1,    // + (gq - 1)
@@ -149,7 +148,6 @@ enum Kern {
     K_GEMM_MFMA16_SWIGLU,
     K_NORM_W,
     K_GEMM_MFMA16_GROUP,
-    K_GEMM_TILED_GROUP,
     K_GEMM_TILED64_GROUP,
     K_GEMM_TILED32_GROUP,
     K_QUANT_GROUP,
@@ -158,7 +156,6 @@ enum Kern {
     K_LM_CERT,
     K_LM_PICK,
     K_NORM4S_R8,
-    K_GEMM_TILED64_S4,
     K_GEMM_TILED32_S4,
     K_EMBED_Q8,
     K_DEQUANT_F16,
@@ -192,7 +189,7 @@ inline const char* const kKernelNames[] = {
     "lgx_k_repack_f16_t64", "lgx_k_lm_head_t64", "lgx_k_rows_to_t16",
     "lgx_k_q8_gemv_grpq4", "lgx_k_q8_gemv_grpq8", "lgx_k_q8_gemv_grpq16",
     "lgx_k_add_rmsnorm_quant4_r8", "lgx_k_add_rmsnorm_quant4_r20",
-    "lgx_k_act_to_t16", "lgx_k_q8_gemm_tiled", "lgx_k_q8_gemm_tiled64", "lgx_k_q8_gemm_tiled32",
+    "lgx_k_act_to_t16", "lgx_k_q8_gemm_tiled64", "lgx_k_q8_gemm_tiled32",
     "lgx_k_attn_prefill_d64_g1", "lgx_k_attn_prefill_d64_g2", "lgx_k_attn_prefill_d64_g3",
     "lgx_k_attn_prefill_d64_g4", "lgx_k_attn_prefill_d64_g5", "lgx_k_attn_prefill_d64_g6",
     "lgx_k_attn_prefill_d64_g7", "lgx_k_attn_prefill_d64_g8",
@@ -201,10 +198,10 @@ inline const char* const kKernelNames[] = {
     "lgx_k_attn_prefill_d128_g7", "lgx_k_attn_prefill_d128_g8",
     "lgx_k_sample_partial", "lgx_k_sample_final",
     "lgx_k_q8_gemm_mfma16_qkv", "lgx_k_q8_gemm_mfma16_swiglu", "lgx_k_add_rmsnorm_quant_w",
-    "lgx_k_q8_gemm_mfma16_group", "lgx_k_q8_gemm_tiled_group", "lgx_k_q8_gemm_tiled64_group",
+    "lgx_k_q8_gemm_mfma16_group", "lgx_k_q8_gemm_tiled64_group",
     "lgx_k_q8_gemm_tiled32_group", "lgx_k_quantize_group", "lgx_k_q8_combine_group",
     "lgx_k_lm_rowconst", "lgx_k_lm_cert", "lgx_k_lm_pick", "lgx_k_add_rmsnorm_quant4s_r8",
-    "lgx_k_q8_gemm_tiled64s4", "lgx_k_q8_gemm_tiled32s4", "lgx_k_embed_q8", "lgx_k_dequant_f16",
+    "lgx_k_q8_gemm_tiled32s4", "lgx_k_embed_q8", "lgx_k_dequant_f16",
     "lgx_k_swiglu_f16",
     "lgx_k_attn_prefill_fast_d64_g1", "lgx_k_attn_prefill_fast_d64_g2", "lgx_k_attn_prefill_fast_d64_g3",
     "lgx_k_attn_prefill_fast_d64_g4", "lgx_k_attn_prefill_fast_d64_g5", "lgx_k_attn_prefill_fast_d64_g6",
@@ -252,7 +249,7 @@ struct lgx_ctx {
     bool gemv_whole = false;      // LGX_GEMV=whole: block dots through LDS, chains after
     int gemm_mt = 0;              // LGX_GEMM_MT: force the M > 1 m-tile width (0: by m)
     int tiled_min = 33;           // LGX_GEMM_TILED_MIN: smallest m through the tiled product
-    int tiled_rows = 0;           // LGX_GEMM_TILED_ROWS: force 128/64/32 activation rows per workgroup
+    int tiled_rows = 0;           // LGX_GEMM_TILED_ROWS: force 64 (or more) / 32 activation rows per workgroup
     int tiled_grp = 0;            // LGX_GEMM_TILED_GRP: force 1/2/4 ranges per group
     int tiled_wpc = 4;            // LGX_GEMM_TILED_WPC: workgroups per CU the automatic group choice keeps
     bool decode_streaming = false; // LGX_DECODE_GEMM=streaming: decode products of m >= 17
@@ -572,16 +569,21 @@ inline lgx_status run_q8(lgx_ctx* c, Kern kern, const lgx_q8_matrix* W, const fl
 
 // Tiled product: activations in T16 tiles (ceil(m/16) of them), group
 // partials part[ceil(nr / grp)][m][n] (canonical subtrees of grp aligned
-// ranges, grp in {1, 2, 4}).  Activation rows per workgroup: 128
-// (K_GEMM_TILED), 64 or 32.  With swiglu = I (W the [gate; up] matrix of
+// ranges, grp in {1, 2, 4}).  Activation rows per workgroup: 64
+// (K_GEMM_TILED64) or 32.  With swiglu = I (W the [gate; up] matrix of
 // 2I rows, I % 32 == 0, one group) the SwiGLU + Q8_0 of the outputs goes to
 // sq (T16) / sd instead of part.
+inline int tiled_rows_of(Kern kern) { return kern == K_GEMM_TILED64 ? 64 : 32; }
 inline int tiled_groups(int k, int grp = LGX_TG_RANGES) { return (nranges_of(k) + grp - 1) / grp; }
+// Grid of the tiled product: each group's tiles in whole eights (one per XCD).
+inline int64_t tiled_grid(const lgx_gemm_tiled_args& a) {
+    return ((int64_t)a.ntn * a.ntm + 7) / 8 * 8 * a.ngroups;
+}
 inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t* xt,
                                const uint16_t* xd, int m, float* part, void* stream,
-                               Kern kern = K_GEMM_TILED, int grp = LGX_TG_RANGES,
+                               Kern kern, int grp = LGX_TG_RANGES,
                                int swiglu = 0, int8_t* sq = nullptr, uint16_t* sd = nullptr) {
-    const int mrows = kern == K_GEMM_TILED ? 128 : kern == K_GEMM_TILED64 ? 64 : 32;
+    const int mrows = tiled_rows_of(kern);
     lgx_gemm_tiled_args a{};
     a.wt = W->qs;
     a.wd = W->d;
@@ -604,29 +606,43 @@ inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
     a.ntn = (int)cdiv(W->n, LGX_TG_N);
     a.ntm = (int)cdiv(m, mrows);
     const int64_t wgs = (int64_t)a.ntn * a.ntm * a.ngroups;
-    if (wgs > INT32_MAX) return fail(LGX_OUT_OF_BOUNDS, "tiled product of %lld workgroups", (long long)wgs);
-    // a grid of at most two workgroups per compute unit runs in stages of 4
+    if (tiled_grid(a) > INT32_MAX)
+        return fail(LGX_OUT_OF_BOUNDS, "tiled product of %lld workgroups", (long long)wgs);
+    // a 32-row grid of at most two workgroups per compute unit runs in stages of 4
     // pairs: half the dependent memory rounds per workgroup (config-4 o_proj,
     // 448 workgroups: 8.8 against 10.1 us; at 576 workgroups, three share some
     // compute units and the 2-pair stages are faster: 11.9 against 12.8 us)
-    if (c->tiled_s4 && wgs <= 2 * (int64_t)c->ncu) {
-        if (kern == K_GEMM_TILED32) kern = K_GEMM_TILED32_S4;
-        else if (kern == K_GEMM_TILED64) kern = K_GEMM_TILED64_S4;
-    }
-    return launch(c, kern, dim3((unsigned)wgs), dim3(256), a, stream);
+    if (c->tiled_s4 && kern == K_GEMM_TILED32 && wgs <= 2 * (int64_t)c->ncu) kern = K_GEMM_TILED32_S4;
+    return launch(c, kern, dim3((unsigned)tiled_grid(a)), dim3(256), a, stream);
 }
-// Tiled kernel for m rows: 128 activation rows per workgroup from m >= 128,
-// else 32, which also beats 64 at m = 64 (LGX_GEMM_TILED_ROWS forces one).
-inline Kern tiled_kernel(const lgx_ctx* c, int m) {
-    const int rows = c->tiled_rows ? c->tiled_rows : m >= 128 ? 128 : 32;
-    return rows == 128 ? K_GEMM_TILED : rows == 64 ? K_GEMM_TILED64 : K_GEMM_TILED32;
+// Tiled kernel for a product of n outputs, reduction k, over m rows: 64
+// activation rows per workgroup (32 x 32 matrix instructions, four waves per
+// SIMD) where that grid fills the device, else 32 rows, whose grid is twice
+// the size.  Measured over 0.5B / 1.5B / 7B-shaped products at 64 to 3072
+// rows: 64 rows take 0.78-0.92 of the 32-row time from 600 workgroups on
+// (9728 x 896 at 512 rows 24.3 against 26.9 us, 17920 x 1536 at 2048 184
+// against 238) and 1.1-1.3 of it on small grids (896 x 896 at 512 rows 12.0
+// against 9.1); below 256 rows, where a weight tile serves few workgroups,
+// from about 1150 (17920 x 1536 at 192 rows, 840: 37.7 against 32.1; 37888 x
+// 3584 at 100 rows, 1184: 75.0 against 84.8).  Long reductions, split into
+// several groups, gain from about 200 workgroups (1536 x 8960 at 192 rows
+// 23.4 against 25.1, 3584 x 18944 at 100 43.1 against 50.5), not at 64 rows
+// and below (35.9 against 35.3).  LGX_GEMM_TILED_ROWS forces one.
+inline int64_t tiled64_wgs(int n, int k, int m) {
+    return (int64_t)cdiv(n, LGX_TG_N) * cdiv(m, 64) * tiled_groups(k);
+}
+inline Kern tiled_kernel(const lgx_ctx* c, int n, int k, int m) {
+    if (c->tiled_rows) return c->tiled_rows >= 64 ? K_GEMM_TILED64 : K_GEMM_TILED32;
+    const int64_t wgs = tiled64_wgs(n, k, m);
+    const bool wide = m > 64 && (tiled_groups(k) > 1 ? wgs >= 200 : wgs >= (m >= 256 ? 600 : 1150));
+    return wide ? K_GEMM_TILED64 : K_GEMM_TILED32;
 }
 // Ranges per group for a product of n outputs, reduction k, over m rows
 // through `kern`: the largest of 4, 2, 1 that still gives four workgroups
 // per compute unit (fewer partials when the grid is full anyway).
 inline int tiled_grp(const lgx_ctx* c, Kern kern, int n, int k, int m) {
     if (c->tiled_grp) return c->tiled_grp;
-    const int mrows = kern == K_GEMM_TILED ? 128 : kern == K_GEMM_TILED64 ? 64 : 32;
+    const int mrows = tiled_rows_of(kern);
     const int64_t tiles = (int64_t)cdiv(n, LGX_TG_N) * cdiv(m, mrows);
     for (int grp = 4; grp > 1; grp >>= 1)
         if (tiles * tiled_groups(k, grp) >= (int64_t)c->tiled_wpc * c->ncu) return grp;

@@ -354,7 +354,6 @@ typedef struct {
 // sd ([m][I/32]), the lgx_k_swiglu_quant operations.
 #define LGX_TG_RANGES 4
 #define LGX_TG_N 64
-#define LGX_TG_M 128
 typedef struct {
     const int8_t* wt;      // T16 weights [n/16][k/64][64][16]
     const uint16_t* wd;    // S16 scales

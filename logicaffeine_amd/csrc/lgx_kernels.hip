@@ -24,6 +24,9 @@
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1574,6 +1577,18 @@ __device__ __forceinline__ void static_for(F&& f) {
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 
+// Direct global->LDS loads (a wave instruction's 64 pieces of 16 or 4 bytes
+// land one after the other at l, which is uniform) that the compiler does not
+// count: it makes every LDS read of a loop wait for those it knows, whichever
+// buffer they fill.  They write no register; publish_lds_loads waits for them.
+__device__ __forceinline__ void load_lds_16(const void* g, lds_void* l) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 : : "s"((uint32_t)(uintptr_t)l), "v"(g) : "memory", "m0");
+}
+__device__ __forceinline__ void load_lds_4(const void* g, lds_void* l) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                 : : "s"((uint32_t)(uintptr_t)l), "v"(g) : "memory", "m0");
+}
 // Barrier that publishes this wave's direct global->LDS loads to the
 // workgroup.  The wait is written out: the compiler waits for such a load
 // where its own wave reads the data, which in a loop may be only after the
@@ -4056,16 +4071,15 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_dequant_f16(const lgx_de
 }
 
 // ---------------------------------------------------------------------------
-// Tiled Q8_0 product (prefill; decode batches of 32 / 64 rows).  Workgroup
-// tile: 64 weight rows (4 row tiles) x 32*WM activation rows (2*WM row
-// tiles) over one group of a.grp aligned ranges (1, 2 or 4).  Four waves;
-// wave (wn, wm) owns weight tiles 2wn, 2wn+1 and activation tiles
-// WM*wm .. WM*wm + WM-1.  Per 64-column pair a wave issues one MFMA
-// i32_16x16x32_i8 per (block, weight tile, activation tile) with the weight
-// tile as A, so lane (r, c) of a result holds weight rows 4c..4c+3 of the
+// Tiled Q8_0 product (prefill; decode batches of 33 rows and more), small
+// grids.  Workgroup tile: 64 weight rows (4 row tiles) x 32 activation rows
+// (2 row tiles) over one group of a.grp aligned ranges (1, 2 or 4).  Four
+// waves; wave (wn, wm) owns weight tiles 2wn, 2wn+1 and activation tile wm.
+// Per 64-column pair a wave issues one MFMA i32_16x16x32_i8 per (block,
+// weight tile) with the weight tile as A, so lane (r, c) of a result holds weight rows 4c..4c+3 of the
 // tile against activation row r; the epilogue runs the canonical chain
 // acc = fmaf((float)s, f32(dw) * f32(dx), acc) of each element, the scale
-// products of a (block, weight tile, activation tile) coming from one rank-1
+// products of a (block, weight tile) coming from one rank-1
 // f16 MFMA (16x16x16) with the same lane layout, so the VALU does two
 // operations per element (convert, fma).  When a
 // range ends its values fold into the group's subtree (a binary counter over
@@ -4075,49 +4089,60 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_dequant_f16(const lgx_de
 // is the tree over all ranges.  A gate|up product in one group can instead
 // finish with SwiGLU + Q8_0 in the workgroup (a.swiglu): its tile slots then
 // pair each gate tile with the up tile of the same columns.
-// Staging: two LDS stages of LGX_TG_S pairs filled by direct global->LDS
+// Staging: two LDS stages of S pairs filled by direct global->LDS
 // loads, 16-byte lanes for the T16 tiles and 4-byte lanes for the scale
 // pairs of a 64-column pair, which land pre-arranged: dw as [pair][64 rows]
-// (the four rows of a lane are one 16-byte read), dx as [pair][r][2*WM
-// tiles] (the WM tiles of a wave are one read).  Every operand of a stage is
+// (the four rows of a lane are one 16-byte read), dx as [pair][r][2 tiles].
+// Every operand of a stage is
 // read into registers before the next stage's loads are issued (the
 // compiler would otherwise wait for those loads before the reads).
 // Workgroup order: physical ids go round-robin over the 8 XCDs; each XCD
-// takes a contiguous run of logical tiles, which walk bands of 8 activation
-// tiles, n-tile by n-tile (activation tile fastest), so the tiles in flight
-// on one XCD share their operands through its L2.
+// takes a contiguous run of every group's tiles, which walk bands of 8
+// activation tiles, n-tile by n-tile (activation tile fastest), so the tiles
+// in flight on one XCD share their operands through its L2.
 // ---------------------------------------------------------------------------
 // S pairs per stage: 2, or 4 for grids of at most two workgroups per compute
 // unit (half the stages, so half the dependent memory rounds)
-template <int WM, int S>
+template <int S>
 struct TgSmem {
     uint4 w[4][S][64];
-    uint4 x[2 * WM][S][64];
+    uint4 x[2][S][64];
     uint32_t dw[S][64];
-    uint32_t dx[S][16 * 2 * WM];
+    uint32_t dx[S][32];
 };
 
-template <int WM, int S = 2>
-__device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, const int P) {
-    constexpr int MTILES = 2 * WM;
-    // two stage buffers as two variables: a direct load into one is known
-    // not to alias reads of the other
-    __shared__ TgSmem<WM, S> sm0, sm1;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int wn = wave & 1, wm = wave >> 1;
-    const int r = lane & 15, c = lane >> 4;
-    // XCD-aware logical id, then (group, band of 8 activation tiles, n tile)
-    const int T = a.ntn * a.ntm * a.ngroups;
-    const int xcd = P & 7, slot = P >> 3;
-    const int q8 = T >> 3, r8 = T & 7;
-    const int id = xcd * q8 + min(xcd, r8) + slot;
-    const int per_g = a.ntn * a.ntm;
-    const int g = id / per_g;
-    const int rem = id - g * per_g;
+// Group and tile of workgroup P: XCD P & 7 takes, of every group, a
+// contiguous run of ceil(tiles / 8) or one less (the runs shifted by one XCD
+// per group), so that each XCD has the same share of the last group, whose
+// ranges may be fewer (whole runs of groups per XCD: 8% more on the longest
+// one for 18944 columns); tiles walk bands of 8 activation tiles, n tile by n
+// tile.  False: no tile (the grid is padded to whole eights).
+__device__ __forceinline__ bool tiled_coords(const lgx_gemm_tiled_args& a, int P, int& g, int& tn, int& tm) {
+    const int per_g = a.ntn * a.ntm, tq = (per_g + 7) >> 3, q8 = per_g >> 3, r8 = per_g & 7;
+    const int slot = P >> 3;
+    g = slot / tq;
+    const int x = ((P & 7) + g) & 7, lt = slot - g * tq;
+    if (lt >= q8 + (x < r8 ? 1 : 0)) return false;
+    const int rem = x * q8 + min(x, r8) + lt;
     const int band = rem / (8 * a.ntn);
     const int bsz = min(8, a.ntm - 8 * band);
     const int loc = rem - band * 8 * a.ntn;
-    const int tn = loc / bsz, tm = 8 * band + (loc - (loc / bsz) * bsz);
+    tn = loc / bsz;
+    tm = 8 * band + (loc - tn * bsz);
+    return true;
+}
+
+template <int S = 2>
+__device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, const int P) {
+    constexpr int MTILES = 2;
+    // two stage buffers as two variables: a direct load into one is known
+    // not to alias reads of the other
+    __shared__ TgSmem<S> sm0, sm1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wn = wave & 1, wm = wave >> 1;
+    const int r = lane & 15, c = lane >> 4;
+    int g, tn, tm;
+    if (!tiled_coords(a, P, g, tn, tm)) return;
     const int tn0 = tn * 4, tm0 = tm * MTILES;
 
     const int np = a.k >> 6, nb = a.k >> 5, nh = (a.k + 511) >> 9;
@@ -4142,14 +4167,14 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
     //   weights: 4 tiles x S pairs, units j = wave + 4i (tile j / S, pair j % S)
     //   activations: MTILES tiles x S pairs, likewise
     //   weight scale pairs: [s][64 rows], one 4-byte lane per row (waves < S)
-    //   activation scale pairs: [s][r][tile], wave instructions j = wave < WM
-    static_assert((S == 2 || S == 4) && WM * S <= 8, "stage layout: scale loads on at most four waves");
+    //   activation scale pairs: [s][r][tile], wave instructions j = wave < S / 2
+    static_assert(S == 2 || S == 4, "stage layout: scale loads on at most four waves");
     const uint32_t off_t16 = lane * 16;
     const uint32_t off_dw = ((uint32_t)wtile(lane >> 4) * nh * 256 + (lane & 15) * 16) * 2;
     const int dxp = (wave * 64 + lane) % (16 * MTILES);            // position within a pair
     const int dx_ml = (dxp % MTILES) * 16 + dxp / MTILES;
     const uint32_t off_dx = (uint32_t)min(tm0 * 16 + dx_ml, a.m - 1) * nb * 2;
-    auto stage = [&](TgSmem<WM, S>& sm, int pair0) {
+    auto stage = [&](TgSmem<S>& sm, int pair0) {
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const int j = wave + 4 * i;
@@ -4171,62 +4196,50 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
             const char* base = (const char*)(a.wd + (b >> 4) * 256 + (b & 15));
             __builtin_amdgcn_global_load_lds((const void*)(base + off_dw), (lds_void*)&sm.dw[wave][0], 4, 0, 0);
         }
-        if (wave < WM * S / 2) {                  // 64 words per instruction, 16*MTILES per pair
-            const int s = (wave * 64 + lane) / (16 * MTILES);   // uniform unless WM == 1
+        if (wave < S / 2) {                       // 64 words per instruction, 32 per pair
+            const int s = (wave * 64 + lane) / (16 * MTILES);
             const char* src = (const char*)(a.xd + 2 * min(pair0 + s, pend - 1)) + off_dx;
             __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(&sm.dx[0][0] + wave * 64), 4, 0, 0);
         }
     };
 
-    float acc[2][WM][4], l0[2][WM][4], l1[2][WM][4];
+    float acc[2][4], l0[2][4], l1[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < WM; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[i][j][v] = l0[i][j][v] = l1[i][j][v] = 0.0f;
+        for (int v = 0; v < 4; ++v) acc[i][v] = l0[i][v] = l1[i][v] = 0.0f;
     int cnt = 0;
 
     // One stage: its products from `cur` while the next stage loads into `nxt`.
-    auto run = [&](int q, TgSmem<WM, S>& cur, TgSmem<WM, S>& nxt) {
+    auto run = [&](int q, TgSmem<S>& cur, TgSmem<S>& nxt) {
         __syncthreads();                          // stage q landed; stage q-1 fully read
-        uint4 A[S][2], B[S][WM];
-        uint32_t DWR[S][2], DX[S][WM];
+        uint4 A[S][2], B[S];
+        uint32_t DWR[S][2], DX[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             A[s][0] = cur.w[2 * wn][s][lane];
             A[s][1] = cur.w[2 * wn + 1][s][lane];
-#pragma unroll
-            for (int j = 0; j < WM; ++j) B[s][j] = cur.x[WM * wm + j][s][lane];
+            B[s] = cur.x[wm][s][lane];
             // weight scale pair of row r of tiles 2wn, 2wn+1 (lanes 16.. read
             // the same rows; their values meet zeros in the scale product)
             DWR[s][0] = cur.dw[s][(2 * wn) * 16 + r];
             DWR[s][1] = cur.dw[s][(2 * wn + 1) * 16 + r];
-            const uint32_t* dxr = &cur.dx[s][r * MTILES + WM * wm];
-            if constexpr (WM == 4) {
-                const uint4 q4 = *(const uint4*)dxr;
-                DX[s][0] = q4.x; DX[s][1] = q4.y; DX[s][2] = q4.z; DX[s][3] = q4.w;
-            } else if constexpr (WM == 2) {
-                const uint2 q2 = *(const uint2*)dxr;
-                DX[s][0] = q2.x; DX[s][1] = q2.y;
-            } else {
-                DX[s][0] = dxr[0];
-            }
+            DX[s] = cur.dx[s][r * MTILES + wm];
         }
         if (q + 1 < nst) stage(nxt, pg0 + S * (q + 1));
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             if (pg0 + S * q + s >= pend) continue;      // workgroup-uniform
-            // product u = (block, weight tile, activation tile); product u + 1
+            // product u = (block, weight tile); product u + 1
             // is issued before the epilogue of u, so the MFMA latency is
             // covered by that epilogue
-            constexpr int NU = 4 * WM;
+            constexpr int NU = 4;
             auto mf = [&](int u) -> v4i {
-                const int blk = u / (2 * WM), i = (u / WM) & 1, j = u % WM;
+                const int blk = u >> 1, i = u & 1;
                 const long av = blk ? (long)(((uint64_t)A[s][i].w << 32) | A[s][i].z)
                                     : (long)(((uint64_t)A[s][i].y << 32) | A[s][i].x);
-                const long bv = blk ? (long)(((uint64_t)B[s][j].w << 32) | B[s][j].z)
-                                    : (long)(((uint64_t)B[s][j].y << 32) | B[s][j].x);
+                const long bv = blk ? (long)(((uint64_t)B[s].w << 32) | B[s].z)
+                                    : (long)(((uint64_t)B[s].y << 32) | B[s].x);
                 return __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, zero, 0, 0, 0);
             };
             // scale products dw[row 4c+v] x dx[row r] of product u as one
@@ -4236,21 +4249,21 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
             // f16 x f16 is exact in binary32 and the zeros make a -0 product
             // +0, which is fmaf(dw, dx, +0) of the canonical epilogue.
             auto sc = [&](int u) -> v4f {
-                const int blk = u / (2 * WM), i = (u / WM) & 1, j = u % WM;
+                const int blk = u >> 1, i = u & 1;
                 // both operands keep only this block's half in lanes 0..15, so
                 // every other term is 0 x 0 (an infinite or NaN scale of the
                 // other block cannot leak in)
                 const uint32_t hm = blk ? 0xffff0000u : 0xffffu;
                 const uint32_t aw = lane < 16 ? DWR[s][i] & hm : 0u;
-                const uint32_t bw = lane < 16 ? DX[s][j] & hm : 0u;
+                const uint32_t bw = lane < 16 ? DX[s] & hm : 0u;
                 const v4h av = __builtin_bit_cast(v4h, make_uint2(aw, 0u));
                 const v4h bv = __builtin_bit_cast(v4h, make_uint2(bw, 0u));
                 return __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, zerof, 0, 0, 0);
             };
             auto ep = [&](int u, const v4i& d, const v4f& sp) {
-                const int i = (u / WM) & 1, j = u % WM;
+                const int i = u & 1;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf((float)d[v], sp[v], acc[i][j][v]);
+                for (int v = 0; v < 4; ++v) acc[i][v] = fmaf((float)d[v], sp[v], acc[i][v]);
             };
             v4i dcur = mf(0);
             v4f scur = sc(0);
@@ -4273,10 +4286,10 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
         if (done % (LGX_Q8_RANGE_BLOCKS / 2) == 0 || q == nst - 1) {
             // range end: fold into the group's subtree (cnt is uniform: one
             // branch per fold)
-            float* A0 = &acc[0][0][0];
-            float* L0 = &l0[0][0][0];
-            float* L1 = &l1[0][0][0];
-            constexpr int NE = 2 * WM * 4;
+            float* A0 = &acc[0][0];
+            float* L0 = &l0[0][0];
+            float* L1 = &l1[0][0];
+            constexpr int NE = 8;
             if (cnt == 0 || cnt == 2) {
 #pragma unroll
                 for (int e = 0; e < NE; ++e) L0[e] = A0[e];
@@ -4299,92 +4312,265 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
         run(q, sm0, sm1);
         if (q + 1 < nst) run(q + 1, sm1, sm0);
     }
-    // the group's value of element (i, j, v)
-    auto fin = [&](int i, int j, int v) {
-        return cnt == 1 ? l0[i][j][v] : cnt == 3 ? l1[i][j][v] + l0[i][j][v] : l1[i][j][v];
+    // the group's value of element (i, v)
+    auto fin = [&](int i, int v) {
+        return cnt == 1 ? l0[i][v] : cnt == 3 ? l1[i][v] + l0[i][v] : l1[i][v];
     };
     if (swi) {
         // SwiGLU + Q8_0 (the lgx_k_swiglu_quant operations on a one-group
         // product): lane (r, c) of wave (w, wm) holds columns 32 tn + 16 w +
-        // 4c .. +3 of activation row r of each tile j; the 32-block of a row
-        // is its four lanes c in both waves w, whose maxima meet in LDS
-        __shared__ float qm_s[2][WM][16][2];
+        // 4c .. +3 of its activation row r; the 32-block of a row is its four
+        // lanes c in both waves w, whose maxima meet in LDS
+        __shared__ float qm_s[2][16][2];
         const int nbl = swi >> 5;
-        float f[WM][4], am[WM];
+        float f[4];
 #pragma unroll
-        for (int j = 0; j < WM; ++j) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) f[j][v] = lgx_silu(fin(0, j, v)) * fin(1, j, v);
-            am[j] = absmax4(f[j]);
-            am[j] = fmaxf(am[j], shfl_xor_f(am[j], 16));
-            am[j] = fmaxf(am[j], shfl_xor_f(am[j], 32));
-            if (c == 0) qm_s[wm][j][r][wn] = am[j];
-        }
+        for (int v = 0; v < 4; ++v) f[v] = lgx_silu(fin(0, v)) * fin(1, v);
+        float am = absmax4(f);
+        am = fmaxf(am, shfl_xor_f(am, 16));
+        am = fmaxf(am, shfl_xor_f(am, 32));
+        if (c == 0) qm_s[wm][r][wn] = am;
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < WM; ++j) {
-            const int m = (tm0 + WM * wm + j) * 16 + r;
-            uint16_t dh;
-            const uint32_t qw = quantize4_am(f[j], fmaxf(qm_s[wm][j][r][0], qm_s[wm][j][r][1]), dh);
-            if (m >= a.m) continue;
-            *(uint32_t*)(a.sq + t16_off(m, 32 * tn + 16 * wn + 4 * c, swi)) = qw;
-            if (wn == 0 && c == 0) a.sd[(int64_t)m * nbl + tn] = dh;
-        }
+        const int m = (tm0 + wm) * 16 + r;
+        uint16_t dh;
+        const uint32_t qw = quantize4_am(f, fmaxf(qm_s[wm][r][0], qm_s[wm][r][1]), dh);
+        if (m >= a.m) return;
+        *(uint32_t*)(a.sq + t16_off(m, 32 * tn + 16 * wn + 4 * c, swi)) = qw;
+        if (wn == 0 && c == 0) a.sd[(int64_t)m * nbl + tn] = dh;
         return;
     }
+    const int m = (tm0 + wm) * 16 + r;
+    if (m >= a.m) return;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int t = tn0 + 2 * wn + i;
         if (t >= ntw) continue;
-        const int n0 = t * 16 + 4 * c;
-#pragma unroll
-        for (int j = 0; j < WM; ++j) {
-            const int m = (tm0 + WM * wm + j) * 16 + r;
-            if (m >= a.m) continue;
-            float f[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) f[v] = fin(i, j, v);
-            *(float4*)(a.part + ((int64_t)g * a.m + m) * a.n + n0) = make_float4(f[0], f[1], f[2], f[3]);
-        }
+        *(float4*)(a.part + ((int64_t)g * a.m + m) * a.n + t * 16 + 4 * c) =
+            make_float4(fin(i, 0), fin(i, 1), fin(i, 2), fin(i, 3));
     }
 }
 
-extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled(const lgx_gemm_tiled_args a) {
-    q8_tiled_body<4>(a, blockIdx.x);
+// The same product over 64 activation rows on 32 x 32 output tiles: one
+// v_mfma_i32_32x32x32_i8 is one block's dots of 1024 outputs and one rank-1
+// v_mfma_f32_32x32x8_f16 their scale products, half the matrix cycles per
+// output of the 16 x 16 forms (9.1 + 8.4 against 17.4 + 17.3 per 256
+// outputs), which leaves the epilogue's convert and fma (VALU, 79% busy) as the
+// bound.  Wave (wn, wm) owns weight rows 32 wn .. + 31 against activation
+// rows 32 wm .. + 31; lane l = row + 32 h of an operand reads the 8-byte
+// chunks 2h and 2h + 1 of its row and block (the same columns for both
+// operands); lane l of a result holds activation row l % 32 and weight rows
+// 8 (i / 4) + 4 (l / 32) + i % 4.  Staging, range folding and order as above.
+// Four waves per SIMD (128 VGPRs) cover the LDS reads and matrix latencies
+// better than prefetching into registers does: 3584 x 18944 at 2048 rows
+// 467 us, against 475 with 128 rows per workgroup at two waves per SIMD and
+// the operands and products one step ahead, 508 with 128 rows and 496 with 64
+// on the 16 x 16 forms; 9728 x 896 at 2048 rows 68 against 76, 86 and 75.
+struct Tg32Smem {
+    uint4 w[4][2][64];
+    uint4 x[4][2][64];
+    uint32_t dw[2][64];
+    uint32_t dx[2][64];
+};
+
+__device__ __forceinline__ void q8_tiled32_body(const lgx_gemm_tiled_args& a, const int P) {
+    constexpr int S = 2;                          // pairs per stage
+    __shared__ Tg32Smem sm0, sm1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wn = wave & 1, wm = wave >> 1;
+    const int r32 = lane & 31, h = lane >> 5;
+    int g, tn, tm;
+    if (!tiled_coords(a, P, g, tn, tm)) return;
+    const int tn0 = tn * 4, tm0 = tm * 4;
+
+    const int np = a.k >> 6, nb = a.k >> 5, nh = (a.k + 511) >> 9;
+    const int ntw = a.n >> 4, ntx = (a.m + 15) >> 4;
+    const int swi = a.swiglu;
+    auto wtile = [&](int s) {
+        return swi ? (s & 1) * (swi >> 4) + 2 * tn + (s >> 1) : min(tn0 + s, ntw - 1);
+    };
+    const int gpairs = a.grp * (LGX_Q8_RANGE_BLOCKS / 2);
+    const int pg0 = g * gpairs;
+    const int pend = min(pg0 + gpairs, np);
+    const int nst = (pend - pg0 + S - 1) / S;
+
+    const uint32_t off_t16 = lane * 16;
+    const uint32_t off_dw = ((uint32_t)wtile(lane >> 4) * nh * 256 + (lane & 15) * 16) * 2;
+    const uint32_t off_dx = (uint32_t)min(tm0 * 16 + lane, a.m - 1) * nb * 2;
+    auto stage = [&](Tg32Smem& sm, int pair0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const int j = wave + 4 * i;
+            const int tile = j / S, s = j - tile * S;
+            const int t = wtile(tile), p = min(pair0 + s, pend - 1);
+            const char* base = (const char*)a.wt + ((int64_t)t * np + p) * 1024;
+            load_lds_16(base + off_t16, (lds_void*)&sm.w[tile][s][0]);
+        }
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const int j = wave + 4 * i;
+            const int tile = j / S, s = j - tile * S;
+            const int t = min(tm0 + tile, ntx - 1), p = min(pair0 + s, pend - 1);
+            const char* base = (const char*)a.xt + ((int64_t)t * np + p) * 1024;
+            load_lds_16(base + off_t16, (lds_void*)&sm.x[tile][s][0]);
+        }
+        if (wave < S) {
+            const int b = 2 * min(pair0 + wave, pend - 1);
+            const char* base = (const char*)(a.wd + (b >> 4) * 256 + (b & 15));
+            load_lds_4(base + off_dw, (lds_void*)&sm.dw[wave][0]);
+        } else {
+            const char* src = (const char*)(a.xd + 2 * min(pair0 + wave - S, pend - 1)) + off_dx;
+            load_lds_4(src, (lds_void*)&sm.dx[wave - S][0]);
+        }
+    };
+    stage(sm0, pg0);
+    // operand byte offsets of blocks 0 and 1; block 1's is opaque to the
+    // compiler, which would otherwise join the blocks' 8-byte chunks into
+    // 16-byte reads and take them apart again with moves (a block's two
+    // chunks are one ds_read2_b64 into its operand registers)
+    int aoff[2], boff[2];
+    aoff[0] = ((2 * wn + (r32 >> 4)) * S * 64 + (r32 & 15) + 32 * h) * 16;
+    boff[0] = ((2 * wm + (r32 >> 4)) * S * 64 + (r32 & 15) + 32 * h) * 16;
+    aoff[1] = aoff[0] + 8;
+    boff[1] = boff[0] + 8;
+    asm volatile("" : "+v"(aoff[1]), "+v"(boff[1]));
+
+    float acc[16], l0[16], l1[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = l0[v] = l1[v] = 0.0f;
+    int cnt = 0;
+
+    // One stage: its products from `cur` while the next stage loads into `nxt`.
+    auto run = [&](int q, Tg32Smem& cur, Tg32Smem& nxt) __attribute__((always_inline)) {
+        publish_lds_loads();                      // stage q landed; stage q-1 fully read
+        if (q + 1 < nst) stage(nxt, pg0 + S * (q + 1));
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            uint2 A[2][2], B[2][2];               // [block][chunk]
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                const uint2* pa = (const uint2*)((const char*)&cur.w[0][s][0] + aoff[blk]);
+                A[blk][0] = pa[0];
+                A[blk][1] = pa[32];
+                const uint2* pb = (const uint2*)((const char*)&cur.x[0][s][0] + boff[blk]);
+                B[blk][0] = pb[0];
+                B[blk][1] = pb[32];
+            }
+            const uint32_t DW = cur.dw[s][32 * wn + r32], DX = cur.dx[s][32 * wm + r32];
+            // scale products as in the 16 x 16 form: only this block's two
+            // scales in slot k = 0 (lanes 0 .. 31), so D = dw x dx + exact
+            // zeros.  A pair past the group's end takes zeros as its scales:
+            // each chain step then adds 0 to a sum that is never -0
+            const uint32_t bits = h == 0 && pg0 + S * q + s < pend ? 16u : 0u;
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                const v4i av = {(int)A[blk][0].x, (int)A[blk][0].y, (int)A[blk][1].x, (int)A[blk][1].y};
+                const v4i bv = {(int)B[blk][0].x, (int)B[blk][0].y, (int)B[blk][1].x, (int)B[blk][1].y};
+                const v16i zero = {};
+                const v16f zerof = {};
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, zero, 0, 0, 0);
+                const v4h aw = __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_ubfe(DW, 16 * blk, bits), 0u));
+                const v4h bx = __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_ubfe(DX, 16 * blk, bits), 0u));
+                const v16f k = __builtin_amdgcn_mfma_f32_32x32x8f16(aw, bx, zerof, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[v] = fmaf((float)d[v], k[v], acc[v]);
+                // one product live at a time
+#pragma unroll
+                for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(acc[v]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const int done = S * (q + 1);
+        if (done % (LGX_Q8_RANGE_BLOCKS / 2) == 0 || q == nst - 1) {
+            if (cnt == 0 || cnt == 2) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) l0[e] = acc[e];
+            } else if (cnt == 1) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) l1[e] = l0[e] + acc[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) l1[e] = l1[e] + (l0[e] + acc[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+            ++cnt;
+        }
+    };
+#pragma unroll 1
+    for (int q = 0;;) {
+        run(q, sm0, sm1);
+        if (++q >= nst) break;
+        run(q, sm1, sm0);
+        if (++q >= nst) break;
+    }
+    auto fin = [&](int v) { return cnt == 1 ? l0[v] : cnt == 3 ? l1[v] + l0[v] : l1[v]; };
+    if (swi) {
+        // SwiGLU + Q8_0: a lane's values 4 e + v (e < 2) are gate columns
+        // 32 tn + 16 wn + 8 e + 4 h + v of its activation row, values
+        // 8 + 4 e + v the up factors; the row's 32-block is the lane pair h
+        // of both waves wn
+        __shared__ float qm_s[2][32][2];
+        const int nbl = swi >> 5;
+        float f[2][4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) f[e][v] = lgx_silu(fin(4 * e + v)) * fin(8 + 4 * e + v);
+        float am = fmaxf(absmax4(f[0]), absmax4(f[1]));
+        am = fmaxf(am, shfl_xor_f(am, 32));
+        if (h == 0) qm_s[wm][r32][wn] = am;
+        publish_lds_loads();                      // (none is in flight here)
+        const int m = tm0 * 16 + 32 * wm + r32;
+        am = fmaxf(qm_s[wm][r32][0], qm_s[wm][r32][1]);
+        uint16_t dh = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t qw = quantize4_am(f[e], am, dh);
+            if (m < a.m) *(uint32_t*)(a.sq + t16_off(m, 32 * tn + 16 * wn + 8 * e + 4 * h, swi)) = qw;
+        }
+        if (m < a.m && wn == 0 && h == 0) a.sd[(int64_t)m * nbl + tn] = dh;
+        return;
+    }
+    const int m = tm0 * 16 + 32 * wm + r32;
+    if (m >= a.m) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = tn0 + 2 * wn + (e >> 1);
+        if (t >= ntw) continue;
+        *(float4*)(a.part + ((int64_t)g * a.m + m) * a.n + t * 16 + 8 * (e & 1) + 4 * h) =
+            make_float4(fin(4 * e), fin(4 * e + 1), fin(4 * e + 2), fin(4 * e + 3));
+    }
 }
-extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled64(const lgx_gemm_tiled_args a) {
-    q8_tiled_body<2>(a, blockIdx.x);
+
+extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lgx_k_q8_gemm_tiled64(const lgx_gemm_tiled_args a) {
+    q8_tiled32_body(a, blockIdx.x);
 }
 extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled32(const lgx_gemm_tiled_args a) {
-    q8_tiled_body<1>(a, blockIdx.x);
-}
-extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled64s4(const lgx_gemm_tiled_args a) {
-    q8_tiled_body<2, 4>(a, blockIdx.x);
+    q8_tiled_body(a, blockIdx.x);
 }
 extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled32s4(const lgx_gemm_tiled_args a) {
-    q8_tiled_body<1, 4>(a, blockIdx.x);
+    q8_tiled_body<4>(a, blockIdx.x);
 }
 // Grouped tiled products (lgx_tiled_group_args): each matrix's workgroups
 // start at a multiple of 8, so the hardware XCD of a workgroup is its
 // within-matrix id's & 7, as the XCD-aware order assumes.
-template <int WM>
+template <int ROWS>
 __device__ __forceinline__ void q8_tiled_group_body(const lgx_tiled_group_args& a) {
     const int bid = blockIdx.x;
     int g = 0;
     while (g + 1 < a.count && bid >= a.wg0[g + 1]) ++g;
     const int P = bid - a.wg0[g];
     const lgx_gemm_tiled_args& m = a.mat[g];
-    if (P >= m.ntn * m.ntm * m.ngroups) return;   // padding to a multiple of 8
-    q8_tiled_body<WM>(m, P);
+    if constexpr (ROWS == 64)
+        q8_tiled32_body(m, P);
+    else
+        q8_tiled_body(m, P);
 }
-extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled_group(const lgx_tiled_group_args a) {
-    q8_tiled_group_body<4>(a);
-}
-extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled64_group(const lgx_tiled_group_args a) {
-    q8_tiled_group_body<2>(a);
+extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lgx_k_q8_gemm_tiled64_group(const lgx_tiled_group_args a) {
+    q8_tiled_group_body<64>(a);
 }
 extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_gemm_tiled32_group(const lgx_tiled_group_args a) {
-    q8_tiled_group_body<1>(a);
+    q8_tiled_group_body<32>(a);
 }
 
 // Q8_0 of several activation matrices in one launch (lgx_quant_group_args):
@@ -4463,8 +4649,6 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // ---------------------------------------------------------------------------
 #define PFA_R 32
 #define PFA_SEG LGX_PFA_SEG
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v32f __attribute__((ext_vector_type(32)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4s lds_v4s;
 

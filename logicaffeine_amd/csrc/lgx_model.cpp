@@ -311,7 +311,7 @@ bool dec_tiled(const lgx_model* md, int m) { return m >= 33 && !md->ctx->decode_
 // against 8.8).  LGX_GEMM_TILED_ROWS forces one width.
 Kern dec_kernel(const lgx_model* md, const DevQ8& W, int m) {
     const lgx_ctx* c = md->ctx;
-    if (c->tiled_rows || m < 49) return tiled_kernel(c, m);
+    if (c->tiled_rows || m < 49) return tiled_kernel(c, W.m.n, W.m.k, m);
     const int64_t tiles32 = cdiv(W.m.n, LGX_TG_N) * cdiv(m, 32);
     const int grp = tiled_grp(c, K_GEMM_TILED32, W.m.n, W.m.k, m);
     return tiles32 * tiled_groups(W.m.k, grp) > 4 * (int64_t)c->ncu ? K_GEMM_TILED64 : K_GEMM_TILED32;
@@ -660,7 +660,8 @@ lgx_status prefill_alloc(lgx_model* md) {
 // Product of W over the chunk's M rows (Q8_0 in T16 tiles pf.xt, scales
 // pf.xd, written so by the producers): group partials of 4 ranges into pf.part.
 lgx_status pf_product(lgx_model* md, const DevQ8& W, int M, void* stream) {
-    return run_q8_tiled(md->ctx, &W.m, md->pf.xt, md->pf.xd, M, md->pf.part, stream);
+    return run_q8_tiled(md->ctx, &W.m, md->pf.xt, md->pf.xd, M, md->pf.part, stream,
+                        tiled_kernel(md->ctx, W.m.n, W.m.k, M));
 }
 
 lgx_status pf_norm(lgx_model* md, const float* w, int M, int n, int nr, bool with_part,
@@ -880,9 +881,10 @@ lgx_status prefill_chunk(lgx_model* md, int B, int n, const int32_t* tokens, int
             return st;
         if (c->tiled_swiglu && I % 32 == 0 && tiled_groups(H) == 1) {
             // SwiGLU + Q8_0 in the gate|up product's workgroups, into pf.sq / pf.sd
-            if ((st = run_q8_tiled(c, &md->gu[l].m, pf.xt, pf.xd, M, pf.part, stream, K_GEMM_TILED,
-                                   LGX_TG_RANGES, I, pf.sq, pf.sd)) != LGX_OK ||
-                (st = run_q8_tiled(c, &md->dn[l].m, pf.sq, pf.sd, M, pf.part, stream)) != LGX_OK)
+            if ((st = run_q8_tiled(c, &md->gu[l].m, pf.xt, pf.xd, M, pf.part, stream,
+                                   tiled_kernel(c, 2 * I, H, M), LGX_TG_RANGES, I, pf.sq, pf.sd)) != LGX_OK ||
+                (st = run_q8_tiled(c, &md->dn[l].m, pf.sq, pf.sd, M, pf.part, stream,
+                                   tiled_kernel(c, H, I, M))) != LGX_OK)
                 return st;
             continue;
         }

@@ -302,6 +302,26 @@ def test_tiled_gemm_small_m_forced(ctx, orc, rows, grp):
         c.close()
 
 
+@pytest.mark.parametrize("n,k,m", [(16, 64, 65), (4608, 1088, 257), (208, 4160, 129), (48, 32768, 66),
+                                   (1040, 18944, 191)])
+def test_tiled64_gemm_edges_bit_exact(orc, n, k, m):
+    """64 activation rows per workgroup at its edges: one weight row tile of
+    four, one 64-column pair, ranges ending mid-stage, a last group of one
+    short range, 32 ranges, activation rows one past a tile."""
+    qs, d = orc.gen_q8_matrix(9, n + k, n, k)
+    x = orc.gen_normal_f32(9, m, (m, k))
+    x[m // 2] = 0.0
+    xq, xd = orc.quantize_q8_0(x)
+    ref = orc.q8_gemm(qs, d, xq, xd)
+    for env in ({}, dict(LGX_GEMM_TILED_ROWS=64), dict(LGX_GEMM_TILED_ROWS=64, LGX_GEMM_TILED_GRP=2)):
+        c = _ctx_with_env(**env)
+        try:
+            y = c.q8_gemm(c.q8_matrix(qs, d), c.to_device(xq), c.to_device(xd))
+            assert np.array_equal(bits(host(y)), bits(ref)), env
+        finally:
+            c.close()
+
+
 @pytest.mark.parametrize("n,k", [(3584, 3584), (1024, 896), (512, 2112), (64, 192), (2048, 18944)])
 @pytest.mark.parametrize("rows", [32, 64])
 def test_tiled_gemm_stage_sizes_agree(orc, n, k, rows):
