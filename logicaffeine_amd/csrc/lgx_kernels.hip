@@ -1536,6 +1536,27 @@ __device__ __forceinline__ float lgx_expf(float x) {
     return p * __uint_as_float((uint32_t)(n + 127) << 23);
 }
 
+// lgx_expf for x <= 0 or NaN: the same operations without the branches that
+// such an x cannot take; the exponent field comes from the low bits of the
+// rounded sum 1.5 * 2^23 + n.
+__device__ __forceinline__ float lgx_expf_nonpos(float x) {
+    const float t = x * 1.44269504088896341f;
+    const float u = t + 12582912.0f;
+    const float nf = u - 12582912.0f;
+    float r = fmaf(-nf, 0.693145751953125f, x);
+    r = fmaf(-nf, 1.42860682030941723e-06f, r);
+    float p = 1.98412698412698413e-04f;
+    p = fmaf(p, r, 1.38888888888888889e-03f);
+    p = fmaf(p, r, 8.33333333333333333e-03f);
+    p = fmaf(p, r, 4.16666666666666667e-02f);
+    p = fmaf(p, r, 1.66666666666666667e-01f);
+    p = fmaf(p, r, 0.5f);
+    p = fmaf(p, r, 1.0f);
+    p = fmaf(p, r, 1.0f);
+    const float e = p * __uint_as_float((__float_as_uint(u) << 23) + 0x3f800000u);
+    return x < -87.33f ? 0.0f : e;
+}
+
 // p of lane J of the lane's 16-lane row (DPP row_newbcast: J is an immediate)
 template <int J>
 __device__ __forceinline__ float row_bcast(int v) {
@@ -1561,21 +1582,26 @@ __device__ __forceinline__ void static_for(F&& f) {
 // read once per group.  Pages: at D = 64 thread t looks up its own token's
 // page (no LDS round or barrier before the K loads), at D = 128 the chunk's
 // 16 entries go through LDS.  Loads: thread t requests its token's whole K
-// row into registers; once it has landed, the workgroup's direct global->LDS
+// row into registers; the workgroup's direct global->LDS
 // loads (global_load_lds_dwordx4, 1 KiB per wave instruction) bring the
 // first 32 KiB of the chunk's V rows into LDS in token order (the whole
 // chunk at D = 64, tokens 0..127 at D = 128; at D = 128 each thread also
 // loads 128 bytes of tokens 128..255 into registers), and V lands while the
-// scores are computed.  Phase 1: thread t runs the canonical score chain
-// over d for the GQ heads (query rows read as workgroup-uniform values).
-// Phase 2: per head the chunk max (exact in any order), p_t =
-// lgx_expf(s_t - m), and the halving-tree sum of the 256 slots.  Phase 3:
-// the canonical chain over the chunk's tokens, o[i] = fmaf(p_t, V_t[i],
-// o[i]), for every (head, i).  Partials (o_c, m_c, l_c) go to `part`;
+// scores are computed.  Phase 1: thread t's token's canonical score chain
+// over d for the GQ heads.  Phase 2: per head the chunk max (exact in any
+// order), p_t = lgx_expf(s_t - m), and the halving-tree sum of the 256 slots.
+// Phase 3: the canonical chain over the chunk's tokens, o[i] = fmaf(p_t,
+// V_t[i], o[i]), for every (head, i).  The chains run on v_mfma_f32_4x4x1
+// (one product added per step and rounded, the bits of fmaf) or on the VALU.
+// Bound by K/V traffic and its latency (64 sequences of up to 4096 tokens, 28/4
+// heads: 74 us for 287 MB, 95 us before with the VALU chains and the same
+// chunk indexes on the same XCD).  Partials (o_c, m_c, l_c) go to `part`;
 // lgx_k_attn_combine merges the chunks.  LDS: 32 KiB of V + 1088 bytes per
 // head.
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
 
 // Direct global->LDS loads (a wave instruction's 64 pieces of 16 or 4 bytes
 // land one after the other at l, which is uniform) that the compiler does not
@@ -1598,6 +1624,14 @@ __device__ __forceinline__ void publish_lds_loads() {
     __syncthreads();
 }
 
+// 16-byte piece slot of piece c of V row t in LDS: at D = 128 the 128-byte
+// halves of odd rows change places, so that the four rows of a transposing
+// load meet no bank twice more than they must.
+template <int D>
+__device__ __forceinline__ int attn_vswz(int t, int c) {
+    return D == 128 ? c ^ ((t & 1) << 3) : c;
+}
+
 // The chunk's first 32 KiB of V rows (KV head g, pages pg_s) into v_s in
 // token order: wave instruction j moves bytes [1024 j, +1024), which lie in
 // page j / (D/32).  Every instruction is issued, so the compiler can count
@@ -1608,16 +1642,28 @@ __device__ __forceinline__ void attn_stage_v(const lgx_attn_args& a, int g, int 
                                              const int* pg_s, uint16_t* v_s, int wave, int lane) {
     constexpr int PER_PAGE = LGX_PAGE * D * 2 / 1024;   // wave instructions per page
     constexpr int NJ = 32768 / 1024;
+    constexpr int CPR = D / 8, TPI = 64 / CPR;          // pieces per row, rows per instruction
 #pragma unroll
     for (int i = 0; i < NJ / 4; ++i) {
         const int j = wave + 4 * i;
         const int u = j / PER_PAGE;
         const int pg = u * LGX_PAGE < n ? pg_s[u] : pg_s[0];
-        const uint16_t* src = a.vpages + ((int64_t)pg * a.hkv + g) * LGX_PAGE * D +
-                              (j - u * PER_PAGE) * 512 + lane * 8;
+        const int t = (j - u * PER_PAGE) * TPI + lane / CPR;
+        const uint16_t* src = a.vpages + (((int64_t)pg * a.hkv + g) * LGX_PAGE + t) * D +
+                              attn_vswz<D>(t, lane % CPR) * 8;
         __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(v_s + j * 512), 16, 0, 0);
     }
 }
+
+// Which chains run on the matrix instruction (4 heads a step).  Measured at 32
+// sequences of 2048 tokens, 4 KV heads (VALU forms / these, us): scores and PV
+// at D = 128: 28.7 / 30.2 with one head per group, 31.8 / 31.0 with two,
+// 35.1 / 32.0 four, 43.6 / 35.8 seven, 48.7 / 36.8 eight.  At D = 64 scores
+// only (PV there has work for two waves of a single dependent chain each):
+// 16.9 / 17.8 with one head, 18.1 / 18.1 two, 20.8 / 19.3 four, 25.2 / 22.5
+// seven, 28.2 / 24.7 eight; PV too 24.8 and 26.2 with seven and eight.
+constexpr bool attn_mfma_scores(int d, int gq) { return gq >= (d == 128 ? 2 : 3); }
+constexpr bool attn_mfma_pv(int d, int gq) { return d == 128 && gq >= 2; }
 
 template <int D, int GQ>
 __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
@@ -1626,26 +1672,50 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     constexpr int NVS = C / VT;                   // V stages: 1 (D = 64) or 2 (D = 128)
     constexpr int CPR = D / 8;                    // 16-byte pieces per row
     constexpr int NVB = NVS > 1 ? VT * CPR / 256 : 1;   // register pieces per thread
+    constexpr int HG = (GQ + 3) / 4;              // head groups of 4
+    constexpr int PS = C + 16, QS = D + 16;       // p and q row strides: neighbouring heads 16 banks apart
+    // chains on the matrix instruction (4 heads per step), else on the VALU
+    constexpr bool MS = attn_mfma_scores(D, GQ);           // scores
+    constexpr bool MP = attn_mfma_pv(D, GQ);           // PV
     static_assert(NVS <= 2 && GQ <= 8, "chunk V in at most two 32 KiB stages, 8 heads");
     __shared__ __align__(16) uint16_t v_s[VT * D];
-    // p rows padded by 16 floats: rows of neighbouring heads start 16 banks apart
-    __shared__ __align__(16) float p_s[GQ][C + 16];
+    __shared__ __align__(16) float p_s[GQ * PS];  // D = 128: the query rows before the scores
     __shared__ float mx_s[GQ][4];
     __shared__ int pg_s[C / LGX_PAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = blockIdx.x, bg = blockIdx.y;
+    // workgroup x of a sequence's row takes chunk (x + row) mod nchunk: ids go
+    // round-robin over the 8 XCDs, and with a multiple of 8 chunks per row an
+    // XCD would otherwise hold the same chunk index of every sequence (few of
+    // which reach the late chunks)
+    const int bg = blockIdx.y, c = (int)((blockIdx.x + blockIdx.y) % gridDim.x);
     const int b = bg / a.hkv, g = bg - b * a.hkv;
-    // one load per 64-byte line of the group's query rows, issued first: the
-    // rows (written by the previous kernel) travel from memory while the
-    // length, pages and K rows do, and the score chain's scalar loads of
-    // them hit the cache
-    const float qpf = tid < GQ * D / 16 ? a.q[((int64_t)b * a.hq + g * GQ) * D + 16 * tid] : 0.0f;
+    const int h0 = g * GQ;
+    // the query rows as the matrix A operand, requested first: lane l of
+    // register j holds dimension 16 j + l / 4 of head l % 4 of a group (heads
+    // past the last repeat it).  D = 64 reads them from memory; D = 128 passes
+    // them through LDS with the page entries.
+    const float* qrow = a.q + ((int64_t)b * a.hq + h0) * D;
+    float qa[HG][D == 64 ? D / 16 : 1];
+    float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    // VALU: one load per 64-byte line of the rows, so that the score chain's
+    // scalar loads of them hit the cache
+    float qpf = 0.0f;
+    if constexpr (!MS) {
+        if (tid < GQ * D / 16) qpf = qrow[16 * tid];
+    } else if constexpr (D == 64) {
+#pragma unroll
+        for (int hg = 0; hg < HG; ++hg)
+#pragma unroll
+            for (int j = 0; j < D / 16; ++j)
+                qa[hg][j] = qrow[min(4 * hg + (lane & 3), GQ - 1) * D + 16 * j + (lane >> 2)];
+    } else {
+        q4 = *(const float4*)(qrow + 4 * min(tid, GQ * D / 4 - 1));
+    }
     const int L = min(a.seq_len[b] + a.len_add, a.maxlen);
     const int t0 = c * C;
     if (t0 >= L) return;                          // whole workgroup: chunk past the end
     const int n = min(C, L - t0);
-    const int h0 = g * GQ;
     // D = 64: every thread looks up its own token's page (the last token's
     // past the end: a real slot, never used), so no LDS round and no barrier
     // stand before the K loads; D = 128 shares the chunk's 16 entries in LDS
@@ -1659,6 +1729,7 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
             if (t0 + tid * LGX_PAGE < L) pg = a.page_table[(int64_t)b * a.maxp + t0 / LGX_PAGE + tid];
             pg_s[tid] = min(max(pg, 0), a.num_pages - 1);
         }
+        if (MS && tid < GQ * D / 4) *(float4*)(p_s + (tid / (D / 4)) * QS + (tid % (D / 4)) * 4) = q4;
         __syncthreads();
         pgt = pg_s[tid >> 4];
     }
@@ -1666,9 +1737,6 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     // phase 1: scores.  Thread t owns token t; its whole K row is requested
     // before the first use so all of its loads are in flight together (the
     // row address is a real page slot for every thread: pg_s is clamped).
-    float s[GQ];
-#pragma unroll
-    for (int h = 0; h < GQ; ++h) s[h] = 0.0f;
     const bool valid = tid < n;
     uint4 kv[CPR];
     {
@@ -1676,13 +1744,17 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
 #pragma unroll
         for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
     }
-    // the K row has arrived before V is requested: the compiler waits for
-    // every outstanding load before the first use of any of them once the
-    // LDS loads are in flight, so V's transfer overlaps the score chain only
-    // when it is requested after K is in registers
+    // D = 128: the K row has arrived before V is requested (once direct loads
+    // are in flight the compiler waits for every load before the first use of
+    // any), so V's transfer overlaps the score chain: 79.2 against 79.9 us for
+    // 64 sequences of up to 4096 tokens.  D = 64, whose grids leave memory idle
+    // at the start, requests both at once (17.2 against 17.7 us for 32
+    // sequences of 2048).
+    if constexpr (D == 128) {
 #pragma unroll
-    for (int j = 0; j < CPR; ++j)
-        asm volatile("" : "+v"(kv[j].x), "+v"(kv[j].y), "+v"(kv[j].z), "+v"(kv[j].w));
+        for (int j = 0; j < CPR; ++j)
+            asm volatile("" : "+v"(kv[j].x), "+v"(kv[j].y), "+v"(kv[j].z), "+v"(kv[j].w));
+    }
     if constexpr (D == 64) {
         // the whole chunk's V (32 KiB): wave w moves its own tokens
         // 64 w .. 64 w + 63 (wave instructions 8 w .. 8 w + 7, two per page),
@@ -1697,7 +1769,7 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     } else {
         attn_stage_v<D>(a, g, n, pg_s, v_s, wave, lane);
     }
-    // D = 128: tokens VT.. of V, piece q = 256 i + tid of the second stage
+    // D = 128: tokens VT.. of V, slot q = 256 i + tid of the second stage
     // (coalesced: 16 lanes per row), stored to v_s after the first stage
     // (rows past the chunk's end read a real page slot: pg_s is clamped)
     u32x4 vb[NVB];
@@ -1707,33 +1779,66 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
         for (int i = 0; i < NVB; ++i) {
             const int q = 256 * i + tid, tk = VT + q / CPR;
             vb[i] = *(const u32x4*)(a.vpages + (((int64_t)pg_s[tk >> 4] * a.hkv + g) * LGX_PAGE + (tk & 15)) * D +
-                                    (q % CPR) * 8);
+                                    attn_vswz<D>(tk, q % CPR) * 8);
         }
     }
-    __builtin_amdgcn_sched_barrier(0);           // keep every load ahead of the FMAs
-    if (valid) {
+    __builtin_amdgcn_sched_barrier(0);           // keep every load ahead of the products
+    float s[GQ];
+    if constexpr (MS) {
+        // v_mfma_f32_4x4x1, 16 blocks of 4 heads x 4 tokens: dimension 16 j + e of
+        // the group's heads (block e of the A register) against lane l's own token
+        // adds one product to each of the lane's four chains
+        v4f sc[HG];
+#pragma unroll
+        for (int hg = 0; hg < HG; ++hg) sc[hg] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        static_for<0, D / 16>([&](auto J) {
+            float qj[HG];
+#pragma unroll
+            for (int hg = 0; hg < HG; ++hg) {
+                if constexpr (D == 64)
+                    qj[hg] = qa[hg][J.value];
+                else
+                    qj[hg] = p_s[min(4 * hg + (lane & 3), GQ - 1) * QS + 16 * J.value + (lane >> 2)];
+            }
+            const uint32_t w8[8] = {kv[2 * J.value].x,     kv[2 * J.value].y,     kv[2 * J.value].z,
+                                    kv[2 * J.value].w,     kv[2 * J.value + 1].x, kv[2 * J.value + 1].y,
+                                    kv[2 * J.value + 1].z, kv[2 * J.value + 1].w};
+            static_for<0, 16>([&](auto E) {
+                constexpr int e = E.value;
+                const float kf = h2f(e & 1 ? w8[e >> 1] >> 16 : w8[e >> 1] & 0xffffu);
+#pragma unroll
+                for (int hg = 0; hg < HG; ++hg)
+                    sc[hg] = __builtin_amdgcn_mfma_f32_4x4x1f32(qj[hg], kf, sc[hg], 4, e, 0);
+            });
+        });
+#pragma unroll
+        for (int h = 0; h < GQ; ++h) s[h] = sc[h >> 2][h & 3];
+    } else {
         // workgroup-uniform query rows through the scalar cache (the LDS
         // loads above would otherwise keep the compiler from proving them
         // read-only and scalar)
-        const __attribute__((address_space(4))) float* qb =
-            (const __attribute__((address_space(4))) float*)(a.q + ((int64_t)b * a.hq + h0) * D);
-        // the heads run in two passes over the K row (fewer query
-        // values live in scalar registers at once); each chain is unchanged
-        constexpr int HP = (GQ + 1) / 2;
-        static_for<0, (GQ + HP - 1) / HP>([&](auto P) {
-            constexpr int hlo = P.value * HP, hhi = hlo + HP < GQ ? hlo + HP : GQ;
 #pragma unroll
-            for (int j = 0; j < CPR; ++j) {
-                const float kf[8] = {h2f(kv[j].x & 0xffffu), h2f(kv[j].x >> 16), h2f(kv[j].y & 0xffffu),
-                                     h2f(kv[j].y >> 16),     h2f(kv[j].z & 0xffffu), h2f(kv[j].z >> 16),
-                                     h2f(kv[j].w & 0xffffu), h2f(kv[j].w >> 16)};
+        for (int h = 0; h < GQ; ++h) s[h] = 0.0f;
+        if (valid) {
+            const __attribute__((address_space(4))) float* qb = (const __attribute__((address_space(4))) float*)qrow;
+            // the heads run in two passes over the K row (fewer query values
+            // live in scalar registers at once); each chain is unchanged
+            constexpr int HP = (GQ + 1) / 2;
+            static_for<0, (GQ + HP - 1) / HP>([&](auto P) {
+                constexpr int hlo = P.value * HP, hhi = hlo + HP < GQ ? hlo + HP : GQ;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
+                for (int j = 0; j < CPR; ++j) {
+                    const float kf[8] = {h2f(kv[j].x & 0xffffu), h2f(kv[j].x >> 16), h2f(kv[j].y & 0xffffu),
+                                         h2f(kv[j].y >> 16),     h2f(kv[j].z & 0xffffu), h2f(kv[j].z >> 16),
+                                         h2f(kv[j].w & 0xffffu), h2f(kv[j].w >> 16)};
 #pragma unroll
-                    for (int h = hlo; h < hhi; ++h) s[h] = fmaf(qb[h * D + 8 * j + e], kf[e], s[h]);
+                    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+                        for (int h = hlo; h < hhi; ++h) s[h] = fmaf(qb[h * D + 8 * j + e], kf[e], s[h]);
+                    }
                 }
-            }
-        });
+            });
+        }
     }
     // phase 2: max, exp, halving-tree sum.  The wave maxima of the heads
     // advance level by level together (independent shuffles in flight at
@@ -1752,14 +1857,13 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
             for (int h = 0; h < GQ; ++h) mx_s[h][wave] = mw[h];
         }
     }
-    __syncthreads();
+    __syncthreads();                             // ... and the query rows are fully read
 #pragma unroll
     for (int h = 0; h < GQ; ++h) {
         const float m = fmaxf(fmaxf(mx_s[h][0], mx_s[h][1]), fmaxf(mx_s[h][2], mx_s[h][3]));
-        p_s[h][tid] = valid ? lgx_expf(s[h] - m) : 0.0f;
+        p_s[h * PS + tid] = valid ? lgx_expf_nonpos(s[h] - m) : 0.0f;
     }
-    __builtin_amdgcn_s_waitcnt(0);               // this wave's first-stage V is in LDS
-    __syncthreads();                             // ... and every other wave's, and p
+    publish_lds_loads();                         // the first V stage, and p, of every wave
     {
         // head h's sum on wave h % 4: levels 128 and 64 of the tree from
         // p_s, the rest across lanes
@@ -1767,7 +1871,8 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
         for (int h0w = 0; h0w < GQ; h0w += 4) {
             const int h = h0w + wave;
             if (h < GQ) {
-                float l = (p_s[h][lane] + p_s[h][lane + 128]) + (p_s[h][lane + 64] + p_s[h][lane + 192]);
+                const float* ph = p_s + h * PS + lane;
+                float l = (ph[0] + ph[128]) + (ph[64] + ph[192]);
                 l = wave_tree_sum(l);
                 if (lane == 0) {
                     const float m = fmaxf(fmaxf(mx_s[h][0], mx_s[h][1]), fmaxf(mx_s[h][2], mx_s[h][3]));
@@ -1778,12 +1883,70 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
             }
         }
     }
-    // phase 3: o_c[i] = chain_t fmaf(p_t, V_t[i], o).  n is
-    // workgroup-uniform, so the loop bounds do not diverge.
-    if constexpr (D == 64) {
-        // thread = (dimension pair, head group) reads its pair of each V
-        // row from LDS (a wave reads whole rows, conflict-free), four
-        // tokens per step with p as one float4
+    // phase 3: o_c[i] = chain_t fmaf(p_t, V_t[i], o)
+    auto second_stage = [&]() __attribute__((always_inline)) {
+        __syncthreads();                          // the first stage is fully read
+#pragma unroll
+        for (int i = 0; i < NVB; ++i) *(u32x4*)(v_s + (256 * i + tid) * 8) = vb[i];
+        __syncthreads();
+    };
+    if constexpr (MP) {
+        // the same instruction, lane l = dimension 64 dg + l, A = p of 16 tokens x 4 heads (one read), B
+        // = V through the transposing LDS load (four tokens of the lane's
+        // dimension each).  A wave runs one head group over 64 dimensions; where
+        // that leaves two of the four waves idle, the chunk's parity picks which.
+        constexpr int DG = D / 64;
+        const int unit = HG * DG <= 2 ? wave ^ ((c & 1) << 1) : wave;
+        const int dg = unit % DG, hg = unit / DG;
+        const bool on = hg < HG;                      // wave-uniform
+        const int qc = lane & 15, kg = lane >> 4;
+        const float* pa = p_s + min(4 * hg + (lane & 3), GQ - 1) * PS + (lane >> 2);
+        v4f o = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        auto pv_stage = [&](int tb) __attribute__((always_inline)) {   // tokens [tb, min(n, tb + VT)) from v_s
+            const int te = min(n, tb + VT);
+            // V of tokens ts + 4 u .. + 3: lane (qc, kg) loads row qc / 4, dimensions
+            // 16 kg + 4 (qc % 4) .. of the 64, and receives dimension 16 kg + qc
+            auto v_at = [&](int ts, int u) {
+                const int t = ts - tb + 4 * u + (qc >> 2);
+                return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_v4s*)(v_s + t * D + attn_vswz<D>(t, 8 * dg + 2 * kg + ((qc >> 1) & 1)) * 8 + (qc & 1) * 4));
+            };
+            int ts = tb;
+            for (; ts + 16 <= te; ts += 16) {
+                const float p16 = pa[ts];
+                v4s vw[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) vw[u] = v_at(ts, u);
+                static_for<0, 16>([&](auto E) {
+                    constexpr int e = E.value;
+                    o = __builtin_amdgcn_mfma_f32_4x4x1f32(p16, h2f((uint16_t)vw[e >> 2][e & 3]), o, 4, e, 0);
+                });
+            }
+            if (ts < te) {                            // the chunk's last tokens one by one
+                const float p16 = pa[ts];
+                static_for<0, 16>([&](auto E) {
+                    constexpr int e = E.value;
+                    if (ts + e < te)
+                        o = __builtin_amdgcn_mfma_f32_4x4x1f32(p16, h2f((uint16_t)v_at(ts, e >> 2)[e & 3]), o, 4, e, 0);
+                });
+            }
+        };
+        if (on) pv_stage(0);
+        if (two) {
+            second_stage();
+            if (on) pv_stage(VT);
+        }
+        if (on) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int h = 4 * hg + i;
+                if (h < GQ)
+                    a.part[(((int64_t)b * a.hq + h0 + h) * a.nchunk + c) * (D + 2) + 64 * dg + lane] = o[i];
+            }
+        }
+    } else {
+        // thread = (dimension pair, head group) reads its pair of each V row
+        // from LDS (a wave reads whole rows, conflict-free), p as float4
         constexpr int NP = D / 2;                 // dimension pairs
         constexpr int NHG = 256 / NP;             // head groups
         constexpr int HPG = (GQ + NHG - 1) / NHG; // heads per group
@@ -1791,65 +1954,53 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
         float o[HPG][2];
 #pragma unroll
         for (int k = 0; k < HPG; ++k) o[k][0] = o[k][1] = 0.0f;
-        const uint32_t* vs = (const uint32_t*)v_s + ip;
-        int t = 0;
-        // 16 tokens per step: every read of the step (V pairs, p as float4)
-        // issued before the chains
-        for (; t + 16 <= n; t += 16) {
-            uint32_t vv[16];
-            float4 p4[HPG][4];
+        auto pv_stage = [&](int tb) __attribute__((always_inline)) {   // tokens [tb, min(n, tb + VT)) from v_s
+            const int te = min(n, tb + VT);
+            auto v_at = [&](int t) {
+                return *((const uint32_t*)(v_s + (t - tb) * D + attn_vswz<D>(t, ip >> 2) * 8) + (ip & 3));
+            };
+            auto steps = [&](int t, auto N) __attribute__((always_inline)) {   // N tokens, every read before the chains
+                constexpr int NT = N.value;
+                uint32_t vv[NT];
+                float pt[HPG][NT];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) vv[u] = vs[(t + u) * NP];
+                for (int u = 0; u < NT; ++u) vv[u] = v_at(t + u);
 #pragma unroll
-            for (int k = 0; k < HPG; ++k) {
-                const int h = min(hg + NHG * k, GQ - 1);
+                for (int k = 0; k < HPG; ++k) {
+                    const float* ph = p_s + min(hg + NHG * k, GQ - 1) * PS + t;
+                    if constexpr (NT % 4 == 0) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) p4[k][q] = *(const float4*)&p_s[h][t + 4 * q];
-            }
+                        for (int u = 0; u < NT; u += 4) {
+                            const float4 p4 = *(const float4*)(ph + u);
+                            pt[k][u] = p4.x;
+                            pt[k][u + 1] = p4.y;
+                            pt[k][u + 2] = p4.z;
+                            pt[k][u + 3] = p4.w;
+                        }
+                    } else {
+                        pt[k][0] = ph[0];
+                    }
+                }
 #pragma unroll
-            for (int k = 0; k < HPG; ++k) {
-                if (hg + NHG * k < GQ) {
+                for (int k = 0; k < HPG; ++k) {
+                    if (hg + NHG * k < GQ) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float pt[4] = {p4[k][q].x, p4[k][q].y, p4[k][q].z, p4[k][q].w};
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            o[k][0] = fmaf(pt[u], h2f(vv[4 * q + u] & 0xffffu), o[k][0]);
-                            o[k][1] = fmaf(pt[u], h2f(vv[4 * q + u] >> 16), o[k][1]);
+                        for (int u = 0; u < NT; ++u) {
+                            o[k][0] = fmaf(pt[k][u], h2f(vv[u] & 0xffffu), o[k][0]);
+                            o[k][1] = fmaf(pt[k][u], h2f(vv[u] >> 16), o[k][1]);
                         }
                     }
                 }
-            }
-        }
-        for (; t + 4 <= n; t += 4) {
-            uint32_t vv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) vv[u] = vs[(t + u) * NP];
-#pragma unroll
-            for (int k = 0; k < HPG; ++k) {
-                const int h = hg + NHG * k;
-                if (h < GQ) {
-                    const float4 p4 = *(const float4*)&p_s[h][t];
-                    const float pt[4] = {p4.x, p4.y, p4.z, p4.w};
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        o[k][0] = fmaf(pt[u], h2f(vv[u] & 0xffffu), o[k][0]);
-                        o[k][1] = fmaf(pt[u], h2f(vv[u] >> 16), o[k][1]);
-                    }
-                }
-            }
-        }
-        for (; t < n; ++t) {
-            const uint32_t v = vs[t * NP];
-#pragma unroll
-            for (int k = 0; k < HPG; ++k) {
-                const int h = hg + NHG * k;
-                if (h < GQ) {
-                    const float pt = p_s[h][t];
-                    o[k][0] = fmaf(pt, h2f(v & 0xffffu), o[k][0]);
-                    o[k][1] = fmaf(pt, h2f(v >> 16), o[k][1]);
-                }
-            }
+            };
+            int t = tb;
+            for (; t + 16 <= te; t += 16) steps(t, IdxC<16>{});
+            for (; t + 4 <= te; t += 4) steps(t, IdxC<4>{});
+            for (; t < te; ++t) steps(t, IdxC<1>{});
+        };
+        pv_stage(0);
+        if (two) {
+            second_stage();
+            pv_stage(VT);
         }
 #pragma unroll
         for (int k = 0; k < HPG; ++k) {
@@ -1860,75 +2011,11 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
                 pp[1] = o[k][1];
             }
         }
-    } else {
-        // D = 128, all four waves: wave w = (head group hgp = w % HGN,
-        // dimension slice dq = w / HGN); 16-lane row rho is head 4 hgp + rho,
-        // lane k owns DL dimensions of the slice.  The row's p_t comes from
-        // lane t%16 of a 16-token register (DPP row_newbcast), V_t from LDS
-        // (a row reads 16 DL consecutive halves, the four rows the same ones).
-        constexpr int HGN = (GQ + 3) / 4;         // head groups of 4
-        constexpr int WPD = 4 / HGN;              // dimension slices
-        constexpr int DL = D / WPD / 16;          // dimensions per lane: 1, 2 or 4
-        const int hgp = wave % HGN, dq = wave / HGN;
-        const int rho = lane >> 4, k = lane & 15;
-        const int h = 4 * hgp + rho, hc = min(h, GQ - 1);
-        const int dcol = dq * (D / WPD) + DL * k;
-        float o[DL];
-#pragma unroll
-        for (int e = 0; e < DL; ++e) o[e] = 0.0f;
-        // a lane's DL halves of V row tl (as 2 words; DL <= 4)
-        auto v_load = [&](int tl) -> uint2 {
-            if constexpr (DL == 4) return *(const uint2*)(v_s + tl * D + dcol);
-            else if constexpr (DL == 2) return make_uint2(*(const uint32_t*)(v_s + tl * D + dcol), 0u);
-            else return make_uint2(v_s[tl * D + dcol], 0u);
-        };
-        auto pv_apply = [&](const uint2 vv, float pb) {
-            const float vf[4] = {h2f(vv.x & 0xffffu), h2f(vv.x >> 16), h2f(vv.y & 0xffffu), h2f(vv.y >> 16)};
-#pragma unroll
-            for (int e = 0; e < DL; ++e) o[e] = fmaf(pb, vf[e], o[e]);
-        };
-        auto pv_token = [&](int tl, float pb) { pv_apply(v_load(tl), pb); };   // tl: row of the V stage
-        auto pv_stage = [&](int tb) {            // tokens [tb, min(n, tb + VT)) from v_s
-            const int te = min(n, tb + VT);
-            for (int ts = tb; ts < te; ts += 16) {
-                // p of the 16 tokens: four 16-byte reads at one address per
-                // 16-lane row (LDS broadcast), no VALU work per token
-                float pt[16];
-                static_for<0, 4>([&](auto Q) {
-                    const float4 p4 = *(const float4*)&p_s[hc][ts + 4 * Q.value];
-                    pt[4 * Q.value] = p4.x;
-                    pt[4 * Q.value + 1] = p4.y;
-                    pt[4 * Q.value + 2] = p4.z;
-                    pt[4 * Q.value + 3] = p4.w;
-                });
-                if (ts + 16 <= te) {
-                    // the 16 rows' reads issued together, then the chains
-                    uint2 vv[16];
-                    static_for<0, 16>([&](auto J) { vv[J.value] = v_load(ts + J.value - tb); });
-                    static_for<0, 16>([&](auto J) { pv_apply(vv[J.value], pt[J.value]); });
-                } else {
-                    static_for<0, 16>([&](auto J) {
-                        if (ts + J.value < te) pv_token(ts + J.value - tb, pt[J.value]);
-                    });
-                }
-            }
-        };
-        pv_stage(0);
-        if (two) {
-            __syncthreads();                      // the first stage is fully read
-#pragma unroll
-            for (int i = 0; i < NVB; ++i) *(u32x4*)(v_s + (256 * i + tid) * 8) = vb[i];
-            __syncthreads();
-            pv_stage(VT);
-        }
-        if (h < GQ) {
-            float* pp = a.part + (((int64_t)b * a.hq + h0 + h) * a.nchunk + c) * (D + 2) + dcol;
-#pragma unroll
-            for (int e = 0; e < DL; ++e) pp[e] = o[e];
-        }
     }
     // the prefetch's value is never used; this keeps its load in the code
-    if (qpf != qpf && a.len_add == 0x7fffffff) a.part[0] = qpf;
+    if constexpr (!MS) {
+        if (qpf != qpf && a.len_add == 0x7fffffff) a.part[0] = qpf;
+    }
 }
 
 // Merge of the chunk partials of one (sequence, query head): M = max m_c,
@@ -4649,29 +4736,6 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // ---------------------------------------------------------------------------
 #define PFA_R 32
 #define PFA_SEG LGX_PFA_SEG
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4s lds_v4s;
-
-// lgx_expf for x <= 0 or NaN: the same operations without the branches that
-// such an x cannot take; the exponent field comes from the low bits of the
-// rounded sum 1.5 * 2^23 + n.
-__device__ __forceinline__ float lgx_expf_nonpos(float x) {
-    const float t = x * 1.44269504088896341f;
-    const float u = t + 12582912.0f;
-    const float nf = u - 12582912.0f;
-    float r = fmaf(-nf, 0.693145751953125f, x);
-    r = fmaf(-nf, 1.42860682030941723e-06f, r);
-    float p = 1.98412698412698413e-04f;
-    p = fmaf(p, r, 1.38888888888888889e-03f);
-    p = fmaf(p, r, 8.33333333333333333e-03f);
-    p = fmaf(p, r, 4.16666666666666667e-02f);
-    p = fmaf(p, r, 1.66666666666666667e-01f);
-    p = fmaf(p, r, 0.5f);
-    p = fmaf(p, r, 1.0f);
-    p = fmaf(p, r, 1.0f);
-    const float e = p * __uint_as_float((__float_as_uint(u) << 23) + 0x3f800000u);
-    return x < -87.33f ? 0.0f : e;
-}
 
 // Column of token t in a p row: the tokens 16 u + 4 e + g, e = 0..3, of one
 // PV operand lane group g side by side.
