@@ -160,49 +160,20 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_repack_t16(const lgx_rep
 }
 
 // ---------------------------------------------------------------------------
-// Q8_0 activation quantisation: one thread per 32-block.
+// Q8_0 activation quantisation, eight lanes per 32-block (quantize4):
 //   amax = max|x|, d = amax/127, id = d ? 1/d : 0, q = clamp(round(x*id)),
 //   stored scale f16(d) (RNE).
+// Coalesced, and eight times the waves of one thread per block: 64 x 3584 took
+// 4.9 us that way, 3.2 so; 2047 x 18944 (194 MB) 38.8 and 37.6.
 // ---------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(256) void lgx_k_quantize_q8_0(const lgx_quant_args a) {
-    const int nb = a.k >> 5;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)a.m * nb) return;
-    const int64_t row = i / nb, b = i - row * nb;
-    const float4* xp = (const float4*)(a.x + row * a.k + b * 32);
-    float v[32];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        float4 f = xp[j];
-        v[4 * j + 0] = f.x;
-        v[4 * j + 1] = f.y;
-        v[4 * j + 2] = f.z;
-        v[4 * j + 3] = f.w;
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        float t = fabsf(v[j]);
-        amax = t > amax ? t : amax;
-    }
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    uint32_t packed[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float q = roundf(v[4 * j + e] * id);
-            q = fminf(fmaxf(q, -127.0f), 127.0f);
-            w |= ((uint32_t)(int32_t)q & 0xffu) << (8 * e);
-        }
-        packed[j] = w;
-    }
-    uint4* qp = (uint4*)(a.qs + row * a.k + b * 32);
-    qp[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    qp[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-    a.d[i] = f2h(d);
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;   // four values each
+    if (i >= (int64_t)a.m * (a.k >> 2)) return;   // whole 8-lane groups
+    const float4 v = ((const float4*)a.x)[i];
+    const float f[4] = {v.x, v.y, v.z, v.w};
+    uint16_t dh;
+    ((uint32_t*)a.qs)[i] = quantize4(f, dh);
+    if ((threadIdx.x & 7) == 0) a.d[i >> 3] = dh;
 }
 
 // Pairwise tree with doubling stride over p[0..g) (s = 1, 2, 4, ...:
