@@ -215,7 +215,7 @@ lgx_status lgx_lm_head_f16_t64(lgx_ctx* c, const float* x, const uint16_t* emb_t
             return st;
         float* part = nr > 1 ? xt + nxt : logits;
         lgx_lmhead_args a{xt, emb_t64, part, m, h, vocab};
-        if ((st = launch(c, K_LM_HEAD_T64, dim3(cdiv(vocab, 64), mc, nr), dim3(64), a, stream)) != LGX_OK)
+        if ((st = launch(c, K_LM_HEAD_T64, lm_head_grid(vocab, m, nr), dim3(64), a, stream)) != LGX_OK)
             return st;
         if (nr == 1) return LGX_OK;
         lgx_combine_args ca{part, logits, (int64_t)m * vocab, nr};

@@ -403,6 +403,11 @@ inline lgx_status launch_norm(lgx_ctx* c, const lgx_norm_args& a, void* stream) 
                       dim3(512), a, stream, 0u);
     return launch(c, K_ADD_RMSNORM_QUANT, dim3(a.m), dim3(LGX_GLUE_NT), a, stream, 0u);
 }
+// Grid of lgx_k_lm_head_t64: 64-row vocabulary groups in eights x 16-row
+// activation groups, ranges along z.
+inline dim3 lm_head_grid(int vocab, int m, int nr) {
+    return dim3(cdiv(vocab, 512) * 8 * cdiv(m, 16), 1, (unsigned)nr);
+}
 inline int argmax_slices(int vocab) { return (vocab + LGX_ARGMAX_SLICE - 1) / LGX_ARGMAX_SLICE; }
 
 // Certified greedy token of a tied binary16 lm_head (m <= LGX_LMC_MAXB rows

@@ -3310,53 +3310,74 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_rows_to_t16(const lgx_t6
 // 1024-column range per blockIdx.z (the sequential fmaf chain over the
 // range's columns) into range partial z ([ranges][m][vocab], the consumers
 // apply the pairwise tree; h <= 1024 is one range, the logit itself).  One
-// wave per (64 vocabulary rows, 16 activation rows, range): lane l owns
-// vocabulary row 64g + l and keeps 16 chains.  The activation comes in T16 column order, so the 16
-// values of one column are one 64-byte scalar load into SGPRs (wave-uniform,
-// no LDS traffic) feeding 16 independent chains; the binary16 units stream
-// in as whole 1 KiB wave loads, LGX_LMT_PF units ahead.
-#define LGX_LMT_PF 4
+// wave per (64 vocabulary rows, 16 activation rows, range), on
+// v_mfma_f32_16x16x1 (four blocks of 16 vocabulary rows; each step adds one
+// rounded product to every chain, the bits of fmaf): lane l holds vocabulary
+// row 64g + l as the B operand; the activation comes in T16 column order, so
+// that 256 contiguous bytes are 4 columns x 16 rows, one A register whose
+// block b (column b of the four) is broadcast in turn.  The binary16 units
+// stream in as whole 1 KiB wave loads, LGX_LMT_PF pairs of units ahead, the
+// activation (L2) one step ahead.
+// Bound by the binary32 matrix rate (33 cycles a column and wave: 59 us for 32
+// rows x 896 x 151936) and the embedding's 272 MB (45 us): 111 us, 119 with
+// the row groups one grid row after the other (the embedding read twice), 165
+// with 16 fmaf chains a lane on the VALU and the activation in scalar
+// registers.
+#define LGX_LMT_PF 2
 extern "C" __global__ __launch_bounds__(64) void lgx_k_lm_head_t64(const lgx_lmhead_args a) {
-    typedef const __attribute__((address_space(4))) float* cfloat_p;
-    const int g = blockIdx.x, lane = threadIdx.x;
-    const int m0 = blockIdx.y * 16, nm = min(16, a.m - m0);
+    // the 16-row groups of one vocabulary group follow each other on one XCD
+    // (ids go round-robin over the 8): the later ones read its rows from L2
+    const int nmg = (a.m + 15) >> 4, slot = blockIdx.x >> 3;
+    const int mg = slot % nmg, g = (slot / nmg) * 8 + (blockIdx.x & 7), lane = threadIdx.x;
+    if (g * 64 >= a.vocab) return;
+    const int m0 = mg * 16, nm = min(16, a.m - m0);
     const int ncg = a.h >> 3;
-    // the range's units (8 columns each): [128 z, min(ncg, 128 z + 128))
-    const int jb = blockIdx.z * 128, je = min(ncg, jb + 128);
+    // the range's steps of 16 columns (two units): [64 z, min(ncg / 2, 64 z + 64))
+    const int jb = blockIdx.z * 64, je = min(ncg >> 1, jb + 64);
     const uint4* ep = (const uint4*)a.emb + (int64_t)g * ncg * 64 + lane;
-    const cfloat_p xt = (cfloat_p)(a.x + (int64_t)blockIdx.y * a.h * 16);
-    float acc[16];
+    const float* xp = a.x + (int64_t)mg * a.h * 16 + lane;
+    v16f acc = {};
+    // every prefetch is issued (the last step is re-requested at the tail) so
+    // that the compiler's wait counts stay exact
+    uint4 e[LGX_LMT_PF][2];
+    float x[4];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    // h % 32 == 0 (host check): whole groups of LGX_LMT_PF units, and every
-    // prefetch is issued (the last unit is re-requested at the tail) so the
-    // compiler's wait counts stay exact
-    uint4 e[LGX_LMT_PF];
-#pragma unroll
-    for (int u = 0; u < LGX_LMT_PF; ++u) e[u] = ep[(jb + u) * 64];
-    for (int j0 = jb; j0 < je; j0 += LGX_LMT_PF) {
-#pragma unroll
-        for (int u = 0; u < LGX_LMT_PF; ++u) {
-            const int j = j0 + u;
-            const uint4 cur = e[u];
-            e[u] = ep[min(j + LGX_LMT_PF, je - 1) * 64];
-            const float ev[8] = {h2f(cur.x & 0xffffu), h2f(cur.x >> 16), h2f(cur.y & 0xffffu),
-                                 h2f(cur.y >> 16),     h2f(cur.z & 0xffffu), h2f(cur.z >> 16),
-                                 h2f(cur.w & 0xffffu), h2f(cur.w >> 16)};
-            const cfloat_p xc = xt + (int64_t)j * 128;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[r] = fmaf(xc[c * 16 + r], ev[c], acc[r]);
-            }
-        }
+    for (int u = 0; u < LGX_LMT_PF; ++u) {
+        const int j = min(jb + u, je - 1);
+        e[u][0] = ep[2 * j * 64];
+        e[u][1] = ep[(2 * j + 1) * 64];
     }
-    const int v = 64 * g + lane;
-    if (v >= a.vocab) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = xp[jb * 256 + 64 * q];
+    for (int j0 = jb; j0 < je; j0 += LGX_LMT_PF) {
+        static_for<0, LGX_LMT_PF>([&](auto U) {
+            constexpr int u = U.value;
+            const int j = j0 + u;
+            const uint4 c0 = e[u][0], c1 = e[u][1];
+            const float xc[4] = {x[0], x[1], x[2], x[3]};
+            const int jn = min(j + LGX_LMT_PF, je - 1), jx = min(j + 1, je - 1);
+            e[u][0] = ep[2 * jn * 64];
+            e[u][1] = ep[(2 * jn + 1) * 64];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = xp[jx * 256 + 64 * q];
+            if (j < je) {                         // uniform: an odd last step
+                const uint32_t w[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+                static_for<0, 16>([&](auto K) {
+                    constexpr int k = K.value;
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(
+                        xc[k >> 2], h2f(k & 1 ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu), acc, 2, k & 3, 0);
+                });
+            }
+        });
+    }
+    // register 4 blk + i: activation row 4 (l / 16) + i, vocabulary row 64 g +
+    // 16 blk + l % 16
     float* lg = a.logits + (int64_t)blockIdx.z * a.m * a.vocab;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        if (r < nm) lg[(int64_t)(m0 + r) * a.vocab + v] = acc[r];
+    for (int i = 0; i < 16; ++i) {
+        const int r = 4 * (lane >> 4) + (i & 3), v = 64 * g + 16 * (i >> 2) + (lane & 15);
+        if (r < nm && v < a.vocab) lg[(int64_t)(m0 + r) * a.vocab + v] = acc[i];
+    }
 }
 
 // Greedy token, in two launches.  Partial: workgroup (slice, row) takes the

@@ -606,7 +606,7 @@ lgx_status head(lgx_model* md, int B, int32_t* next, void* stream) {
         // [nr][B][vocab], the argmax / draw applies the tree
         nr = nranges_of(H);
         lgx_lmhead_args la{md->xt, md->emb_t64, md->logits, B, H, cf.vocab};
-        if ((st = launch(c, K_LM_HEAD_T64, dim3(cdiv(cf.vocab, 64), cdiv(B, 16), nr), dim3(64), la,
+        if ((st = launch(c, K_LM_HEAD_T64, lm_head_grid(cf.vocab, B, nr), dim3(64), la,
                          stream)) != LGX_OK)
             return st;
         lg = md->logits;
@@ -1455,7 +1455,7 @@ lgx_status lgx_qwen_logits(lgx_model* m, int32_t B, float* out, void* stream) {
             // the certified pick left no logits: the exact lm_head of the
             // step's final-norm rows (still in xt) first
             lgx_lmhead_args la{m->xt, m->emb_t64, m->logits, B, m->c.hidden, m->c.vocab};
-            if ((st = launch(m->ctx, K_LM_HEAD_T64, dim3(cdiv(m->c.vocab, 64), cdiv(B, 16), 1),
+            if ((st = launch(m->ctx, K_LM_HEAD_T64, lm_head_grid(m->c.vocab, B, 1),
                              dim3(64), la, stream)) != LGX_OK)
                 return st;
         }
