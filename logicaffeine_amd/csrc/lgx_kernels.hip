@@ -163,8 +163,9 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_repack_t16(const lgx_rep
 // Q8_0 activation quantisation, eight lanes per 32-block (quantize4):
 //   amax = max|x|, d = amax/127, id = d ? 1/d : 0, q = clamp(round(x*id)),
 //   stored scale f16(d) (RNE).
-// Coalesced, and eight times the waves of one thread per block: 64 x 3584 took
-// 4.9 us that way, 3.2 so; 2047 x 18944 (194 MB) 38.8 and 37.6.
+// Coalesced, and eight times the waves of one thread per block: 64 x 3584 with
+// the product after it 57.9 against 59.2 us; 2047 x 18944 (194 MB) 37.6
+// against 38.8.
 // ---------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(256) void lgx_k_quantize_q8_0(const lgx_quant_args a) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;   // four values each
@@ -3963,24 +3964,40 @@ __device__ __forceinline__ float key_value(uint64_t k) {
     u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
     return __uint_as_float(u);
 }
+// Maximum over the wave in every lane, by lane moves on the VALU.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    auto dpp = [](uint32_t x, auto CTRL) {
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL.value, 0xf, 0xf, false);
+    };
+    v = max(v, dpp(v, IdxC<0xB1>{}));
+    v = max(v, dpp(v, IdxC<0x4E>{}));
+    v = max(v, dpp(v, IdxC<0x141>{}));
+    v = max(v, dpp(v, IdxC<0x140>{}));
+    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max((uint32_t)b[0], (uint32_t)b[1]);
+    const auto c = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max((uint32_t)c[0], (uint32_t)c[1]);
+}
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t k) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)k, o, 64), hi = __shfl_xor((uint32_t)(k >> 32), o, 64);
-        const uint64_t ok = ((uint64_t)hi << 32) | lo;
-        k = ok > k ? ok : k;
-    }
-    return k;
+    const uint32_t hi = wave_max_u32((uint32_t)(k >> 32));
+    const uint32_t lo = wave_max_u32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
+    return ((uint64_t)hi << 32) | lo;
 }
 
 // Slice (4096 logits) x row: each wave takes the top_k keys of its 1024
-// logits by rounds of wave maxima; thread 0 merges the four sorted lists.
+// logits by rounds of wave maxima; the four sorted lists are merged by rank.
+// A lane's 16 logits are kept as the keys' upper halves (the lower half is
+// the index, which lane and register imply), so a round is 32-bit lane moves
+// and compares; lanes with equal values settle by index.  Bound by the rounds
+// (latency and VALU): 32 rows x 151936, top_k = 20: 24.3 us, 37.4 with 64-bit
+// keys, shuffles and the merge on one thread.
 extern "C" __global__ __launch_bounds__(256) void lgx_k_sample_partial(const lgx_sample_args a) {
     __shared__ uint64_t lst[4][LGX_SAMPLE_MAX_K];
+    __shared__ uint64_t merged[LGX_SAMPLE_MAX_K];
     const int sl = blockIdx.x, b = blockIdx.y, t = threadIdx.x, w = t >> 6, l = t & 63;
     const int64_t stride = (int64_t)a.m * a.vocab;
     const int v0 = sl * LGX_ARGMAX_SLICE + w * 1024 + l;
-    uint64_t k[16];
+    uint32_t k[16];
 #pragma unroll
     for (int c = 0; c < 16; c += 4) {
         bool on[4];
@@ -3989,45 +4006,64 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_sample_partial(const lgx
         for (int e = 0; e < 4; ++e) on[e] = v0 + 64 * (c + e) < a.vocab;
         tree_partials_n<4, 8>(a.part, a.nr, stride, (int64_t)b * a.vocab + v0 + 64 * c, 64, on, x);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) k[c + e] = on[e] ? sample_key(x[e], v0 + 64 * (c + e)) : 0;
+        for (int e = 0; e < 4; ++e) k[c + e] = on[e] ? (uint32_t)(sample_key(x[e], 0) >> 32) : 0u;
     }
-    uint64_t lm = 0;
+    if (t < LGX_SAMPLE_MAX_K) merged[t] = 0;
+    // the lane's largest value and the first register that holds it
+    uint32_t lm = 0;
+    int li = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) lm = k[i] > lm ? k[i] : lm;
+    for (int i = 0; i < 16; ++i) {
+        li = k[i] > lm ? i : li;
+        lm = max(lm, k[i]);
+    }
     for (int r = 0; r < a.top_k; ++r) {
-        const uint64_t best = wave_max_u64(lm);
-        if (l == 0) lst[w][r] = best;
+        const uint32_t best = wave_max_u32(lm);
         if (best == 0) {
-            for (int q = r + 1 + l; q < a.top_k; q += 64) lst[w][q] = 0;
+            for (int q = r + l; q < a.top_k; q += 64) lst[w][q] = 0;
             break;                                   // wave-uniform
         }
-        if (lm == best) {                            // keys are unique: one lane
+        const uint64_t tied = __builtin_amdgcn_ballot_w64(lm == best);
+        bool mine = lm == best;
+        if (tied & (tied - 1)) {                     // uniform: the lowest index of the tied lanes
+            const uint32_t first = 1023u - wave_max_u32(mine ? 1023u - (uint32_t)(64 * li + l) : 0u);
+            mine = mine && (uint32_t)(64 * li + l) == first;
+        }
+        if (mine) {
+            lst[w][r] = ((uint64_t)best << 32) | (uint64_t)(0xffffffffu - (uint32_t)(v0 + 64 * li));
             lm = 0;
+            int ni = 0;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                k[i] = k[i] == best ? 0 : k[i];
-                lm = k[i] > lm ? k[i] : lm;
+                k[i] = i == li ? 0u : k[i];
+                ni = k[i] > lm ? i : ni;
+                lm = max(lm, k[i]);
             }
+            li = ni;
         }
     }
     __syncthreads();
-    if (t == 0) {
-        int h[4] = {0, 0, 0, 0};
-        uint64_t* out = a.cand + ((int64_t)b * a.nslices + sl) * LGX_SAMPLE_MAX_K;
-        for (int r = 0; r < a.top_k; ++r) {
-            int wi = 0;
-            uint64_t best = 0;
-            for (int q = 0; q < 4; ++q) {
-                const uint64_t c = h[q] < a.top_k ? lst[q][h[q]] : 0;
-                if (c > best) {
-                    best = c;
-                    wi = q;
+    // an entry's rank: its place in its own list and the larger keys of the
+    // others (each list sorted, keys distinct, 0 for empty places)
+    if (t < 4 * a.top_k) {
+        const int q = t / a.top_k, r = t - q * a.top_k;
+        const uint64_t key = lst[q][r];
+        if (key) {
+            int rank = r;
+            for (int o = 1; o < 4; ++o) {
+                const uint64_t* ol = lst[(q + o) & 3];
+                int lo = 0, hi = a.top_k;            // first place not larger than key
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (ol[mid] > key) lo = mid + 1; else hi = mid;
                 }
+                rank += lo;
             }
-            out[r] = best;
-            if (best) ++h[wi];
+            if (rank < a.top_k) merged[rank] = key;
         }
     }
+    __syncthreads();
+    if (t < a.top_k) a.cand[((int64_t)b * a.nslices + sl) * LGX_SAMPLE_MAX_K + t] = merged[t];
 }
 
 __device__ __forceinline__ uint64_t sm_mix(uint64_t z) {
@@ -4037,60 +4073,65 @@ __device__ __forceinline__ uint64_t sm_mix(uint64_t z) {
 }
 
 // Row b: the top_k keys of the slice lists (rounds of wave maxima over the
-// list heads), then on lane 0, in key order j = 0, 1, ...:
+// list heads, the lists in LDS), then, in key order j = 0, 1, ... (lane j):
 //   e_j = lgx_expf((v_j - v_0) * inv_temp), c_j = c_{j-1} + e_j (c_{-1} = 0)
 //   J   = first j with c_j >= top_p * c_{n-1}
 //   u   = (x >> 40) * 2^-24, x = element pos of stream stream0 + b of seed
 //   pick the first j <= J with c_j > u * c_J (J if none)
+// Latency-bound (one wave per row): the list heads read from memory round by
+// round and the draw on one lane took 20.9 us for 32 rows and top_k = 20, this
+// 12.4.
 extern "C" __global__ __launch_bounds__(64) void lgx_k_sample_final(const lgx_sample_args a) {
-    __shared__ uint64_t top[LGX_SAMPLE_MAX_K];
+    __shared__ uint64_t ls[64 * (LGX_SAMPLE_MAX_K + 1)];
+    __shared__ float es[LGX_SAMPLE_MAX_K];
     const int b = blockIdx.x, l = threadIdx.x;
     const uint64_t* lists = a.cand + (int64_t)b * a.nslices * LGX_SAMPLE_MAX_K;
+    const int pos = a.pos ? a.pos[b] : a.seq_len[b];
+    // list s at ls + s * (top_k + 1): the heads of the lanes' lists spread
+    // over the banks, an empty key behind each list
+    const int ld = a.top_k + 1;
+    for (int i = l; i < a.nslices * a.top_k; i += 64) {
+        const int s = i / a.top_k, r = i - s * a.top_k;
+        ls[s * ld + r] = lists[(int64_t)s * LGX_SAMPLE_MAX_K + r];
+    }
+    __syncthreads();
     int h = 0;
-    uint64_t head = l < a.nslices ? lists[(int64_t)l * LGX_SAMPLE_MAX_K] : 0;
+    uint64_t head = l < a.nslices ? ls[l * ld] : 0, mine = 0;
     int n = 0;
     for (int r = 0; r < a.top_k; ++r) {
         const uint64_t best = wave_max_u64(head);
         if (best == 0) break;                        // wave-uniform
-        if (l == 0) top[r] = best;
+        mine = l == r ? best : mine;                 // lane j keeps key j
         n = r + 1;
         if (head == best) {
             ++h;
-            head = h < a.top_k ? lists[(int64_t)l * LGX_SAMPLE_MAX_K + h] : 0;
+            head = h < a.top_k ? ls[l * ld + h] : 0;
         }
     }
-    __syncthreads();
-    if (l != 0) return;
     int tok = 0;
-    const int pos = a.pos ? a.pos[b] : a.seq_len[b];
     if (n > 0) {
-        const float v0 = key_value(top[0]);
-        float c[LGX_SAMPLE_MAX_K];
-        float acc = 0.0f;
+        const float v0 = key_value(((uint64_t)__builtin_amdgcn_readlane((int)(mine >> 32), 0) << 32));
+        es[l] = l < n ? lgx_expf((key_value(mine) - v0) * a.inv_temp) : 0.0f;
+        __syncthreads();
+        // the running sums in key order, lane j keeping c_j
+        float acc = 0.0f, c = 0.0f;
         for (int j = 0; j < n; ++j) {
-            acc = acc + lgx_expf((key_value(top[j]) - v0) * a.inv_temp);
-            c[j] = acc;
+            acc = acc + es[j];
+            c = l == j ? acc : c;
         }
         const float thr = a.top_p * acc;
-        int J = n - 1;
-        for (int j = 0; j < n; ++j)
-            if (c[j] >= thr) {
-                J = j;
-                break;
-            }
+        const uint64_t reach = __builtin_amdgcn_ballot_w64(l < n && c >= thr);
+        const int J = reach ? __builtin_ctzll(reach) : n - 1;
         const uint64_t sb = sm_mix(a.seed + 0x9E3779B97F4A7C15ull) ^
                             sm_mix(((uint64_t)(a.stream0 + b) + 1ull) * 0xD1B54A32D192ED03ull);
         const uint64_t x = sm_mix(sb + ((uint64_t)pos + 1ull) * 0x9E3779B97F4A7C15ull);
         const float u = (float)(uint32_t)(x >> 40) * 0x1.0p-24f;
-        const float r = u * c[J];
-        int pick = J;
-        for (int j = 0; j <= J; ++j)
-            if (c[j] > r) {
-                pick = j;
-                break;
-            }
-        tok = (int)(0xffffffffu - (uint32_t)top[pick]);
+        const float r = u * __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), J));
+        const uint64_t over = __builtin_amdgcn_ballot_w64(l <= J && c > r);
+        const int pick = over ? __builtin_ctzll(over) : J;
+        tok = (int)(0xffffffffu - (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, pick));
     }
+    if (l != 0) return;
     a.tokens[b] = tok;
     if (a.seq_len) a.seq_len[b] += a.advance;
 }
