@@ -1684,23 +1684,26 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     } else {
         q4 = *(const float4*)(qrow + 4 * min(tid, GQ * D / 4 - 1));
     }
-    const int L = min(a.seq_len[b] + a.len_add, a.maxlen);
     const int t0 = c * C;
+    const int pge = a.page_table[(int64_t)b * a.maxp +
+                                 min(D == 64 ? (t0 + tid) / LGX_PAGE : t0 / LGX_PAGE + (tid & 15), a.maxp - 1)];
+    const int L = min(a.seq_len[b] + a.len_add, a.maxlen);
     if (t0 >= L) return;                          // whole workgroup: chunk past the end
     const int n = min(C, L - t0);
-    // D = 64: every thread looks up its own token's page (the last token's
-    // past the end: a real slot, never used), so no LDS round and no barrier
-    // stand before the K loads; D = 128 shares the chunk's 16 entries in LDS
-    int pgt = 0;
+    // D = 64: every thread looks up its own token's page, so no LDS round and
+    // no barrier stand before the K loads; D = 128 shares the chunk's 16
+    // entries in LDS.  The entries were requested with the length; a token
+    // past the end reads a real slot that the wave (D = 64: lane 0's) or the
+    // pool (D = 128: page 0) has anyway, never used.
+    const bool valid = tid < n;
+    int pgt = 0, slot = tid & 15;
     if constexpr (D == 64) {
-        pgt = a.page_table[(int64_t)b * a.maxp + (t0 + min(tid, n - 1)) / LGX_PAGE];
-        pgt = min(max(pgt, 0), a.num_pages - 1);
+        pgt = min(max(pge, 0), a.num_pages - 1);
+        const int pg0 = __builtin_amdgcn_readfirstlane(pgt);
+        pgt = valid ? pgt : pg0;
+        slot = valid ? slot : 0;
     } else {
-        if (tid < C / LGX_PAGE) {
-            int pg = 0;
-            if (t0 + tid * LGX_PAGE < L) pg = a.page_table[(int64_t)b * a.maxp + t0 / LGX_PAGE + tid];
-            pg_s[tid] = min(max(pg, 0), a.num_pages - 1);
-        }
+        if (tid < C / LGX_PAGE) pg_s[tid] = tid * LGX_PAGE < n ? min(max(pge, 0), a.num_pages - 1) : 0;
         if (MS && tid < GQ * D / 4) *(float4*)(p_s + (tid / (D / 4)) * QS + (tid % (D / 4)) * 4) = q4;
         __syncthreads();
         pgt = pg_s[tid >> 4];
@@ -1709,10 +1712,9 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     // phase 1: scores.  Thread t owns token t; its whole K row is requested
     // before the first use so all of its loads are in flight together (the
     // row address is a real page slot for every thread: pg_s is clamped).
-    const bool valid = tid < n;
     uint4 kv[CPR];
     {
-        const uint4* kr = (const uint4*)(a.kpages + (((int64_t)pgt * a.hkv + g) * LGX_PAGE + (tid & 15)) * D);
+        const uint4* kr = (const uint4*)(a.kpages + (((int64_t)pgt * a.hkv + g) * LGX_PAGE + slot) * D);
 #pragma unroll
         for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
     }
