@@ -245,7 +245,11 @@ def _check(status: int) -> None:
 
 
 def _stream(torch, device):
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """hipStream_t of torch's current stream on `device`, as an integer.  The
+    raw query (0.07 us) where torch has it: building the Stream object of
+    torch.cuda.current_stream takes 2 us of a 7.3 us call."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(device.index) if raw else torch.cuda.current_stream(device).cuda_stream
 
 
 class Q8Matrix:
