@@ -168,13 +168,15 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_repack_t16(const lgx_rep
 // against 38.8.
 // ---------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(256) void lgx_k_quantize_q8_0(const lgx_quant_args a) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;   // four values each
-    if (i >= (int64_t)a.m * (a.k >> 2)) return;   // whole 8-lane groups
-    const float4 v = ((const float4*)a.x)[i];
-    const float f[4] = {v.x, v.y, v.z, v.w};
-    uint16_t dh;
-    ((uint32_t*)a.qs)[i] = quantize4(f, dh);
-    if ((threadIdx.x & 7) == 0) a.d[i >> 3] = dh;
+    const int64_t n = (int64_t)a.m * (a.k >> 2);   // four values each
+    // The grid is capped (LGX_QUANT_WGS); whole 8-lane groups end together.
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const float4 v = ((const float4*)a.x)[i];
+        const float f[4] = {v.x, v.y, v.z, v.w};
+        uint16_t dh;
+        ((uint32_t*)a.qs)[i] = quantize4(f, dh);
+        if ((threadIdx.x & 7) == 0) a.d[i >> 3] = dh;
+    }
 }
 
 // Pairwise tree with doubling stride over p[0..g) (s = 1, 2, 4, ...:

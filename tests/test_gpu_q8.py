@@ -58,6 +58,21 @@ def test_quantize_bit_exact(ctx, orc, m, k):
     assert np.array_equal(u16(d), rd)
 
 
+def test_quantize_more_values_than_one_pass_of_the_grid(ctx, orc):
+    """2^18 workgroups take 2^28 values a pass: the rows on both sides of the
+    first pass's end, and the last, against the oracle."""
+    m, k = 8195, 32768
+    x = ctx.torch.zeros(m, k, dtype=ctx.torch.float32, device=ctx.dev)
+    rows = [0, 8191, 8192, 8194]
+    xr = orc.gen_normal_f32(1, 77, (len(rows), k))
+    x[rows] = ctx.to_device(xr)
+    qs, d = ctx.quantize_q8_0(x)
+    rq, rd = orc.quantize_q8_0(xr)
+    assert np.array_equal(host(qs[rows]), rq)
+    assert np.array_equal(u16(d[rows]), rd)
+    assert not qs[1:8191].any() and not qs[8193].any()
+
+
 def test_quantize_golden_edges(ctx, golden):
     qs, d = ctx.quantize_q8_0(ctx.to_device(golden["edge_x"]))
     assert np.array_equal(host(qs), golden["edge_q"])
