@@ -179,7 +179,9 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* ctx, int32_t count, const lgx_q8_
  * device array of LGX_NOALLOC_SCRATCH_BYTES that the library holds on each
  * device until the process ends; the call allocates nothing and never uses
  * per-kernel timing events.  A product whose intermediates exceed the
- * array fails with LGX_OUT_OF_BOUNDS.  All calls on one device share the
+ * array fails with LGX_OUT_OF_BOUNDS (from 33 rows on they are the T16 copy,
+ * m rounded up to 16 rows x k bytes, and, for k > 4096, ceil(k / 4096) * m * n
+ * binary32 partials at least).  All calls on one device share the
  * array: calls that overlap on one device (two streams, two threads, two
  * ctxs) race. */
 #define LGX_NOALLOC_SCRATCH_BYTES (32u << 20)

@@ -518,12 +518,19 @@ static lgx_status q8_gemm_impl(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
         // T16 copy of the activations, then the group partials (straight
         // into y when K is one group) and the tree over the groups
         const Kern kern = tiled_kernel(c, W->n, W->k, m);
-        const int grp = tiled_grp(c, kern, W->n, W->k, m);
-        const int ng = tiled_groups(W->k, grp);
+        int grp = tiled_grp(c, kern, W->n, W->k, m);
         const size_t xbytes = ((size_t)cdiv(m, 16) * 16 * W->k + 255) / 256 * 256;
+        auto bytes = [&](int g) {
+            const int ng = tiled_groups(W->k, g);
+            return xbytes + (ng > 1 ? (size_t)ng * m * W->n * 4 : 0);
+        };
+        // in a fixed scratch, larger range groups (fewer partials, the same
+        // bits) before the product is refused: 6400 x 18944 at 127 rows needs
+        // 34.9 MB in groups of 2 and 18.7 in groups of 4
+        while (scratch && grp < 4 && bytes(grp) > cap) grp *= 2;
+        const int ng = tiled_groups(W->k, grp);
         float* ws = nullptr;
-        if ((st = room(xbytes + (ng > 1 ? (size_t)ng * m * W->n * 4 : 0), &ws)) != LGX_OK)
-            return st;
+        if ((st = room(bytes(grp), &ws)) != LGX_OK) return st;
         int8_t* xt = (int8_t*)ws;
         float* part = ng > 1 ? (float*)((char*)ws + xbytes) : y;
         if ((st = act_to_t16(c, xq, m, W->k, xt, stream)) != LGX_OK ||

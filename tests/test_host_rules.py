@@ -1,0 +1,85 @@
+"""The host side of the library without a device: which kernels a call
+launches, with which grids, and which calls it refuses.  A child process loads
+tests/hip_stub.cpp (a recording stand-in for the HIP runtime) before liblgx.so
+and runs the calls on made-up pointers."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PTR = 1 << 41                     # any non-NULL device address: nothing runs
+
+CHILD = r"""
+import ctypes as C, json, sys
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+stub.stub_log.restype = C.c_char_p
+import logicaffeine_amd as lgx
+L = lgx.lib()
+h = C.c_void_p()
+lgx._check(L.lgx_ctx_create(0, b"stub", C.byref(h)))
+P = 1 << 41
+for line in sys.stdin:
+    name, args = json.loads(line)
+    def arg(a):
+        if isinstance(a, dict):
+            return C.byref(lgx.Q8MatrixC(P, P, a["n"], a["k"], lgx.Q8_T16))
+        if isinstance(a, list) and a and isinstance(a[0], dict):
+            return (lgx.Q8MatrixC * len(a))(*[lgx.Q8MatrixC(P, P, w["n"], w["k"], lgx.Q8_T16) for w in a])
+        if isinstance(a, list):
+            return (C.c_void_p * len(a))(*a)
+        return a
+    stub.stub_reset()
+    st = getattr(L, name)(h, *[arg(a) for a in args])
+    print(json.dumps([lgx.STATUS_NAMES.get(st, st), stub.stub_log().decode().splitlines()]), flush=True)
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    """calls -> [(status, [kernel launches as (name, gx, gy, gz, block)], bytes allocated)]"""
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", f"-I{rocm}/include", "-o", so,
+                    os.path.join(ROOT, "tests", "hip_stub.cpp")], check=True)
+
+    def run(calls, **env):
+        r = subprocess.run([sys.executable, "-c", CHILD, so], cwd=ROOT, text=True, capture_output=True, timeout=300,
+                           input="".join(json.dumps(c) + "\n" for c in calls), env={**os.environ, **env})
+        assert r.returncode == 0, r.stderr[-4000:]
+        out = []
+        for line in r.stdout.splitlines():
+            st, log = json.loads(line)
+            words = [ln.split() for ln in log]
+            out.append((st, [(w[0], *map(int, w[1:])) for w in words if w[0] != "malloc"],
+                        sum(int(w[1]) for w in words if w[0] == "malloc")))
+        assert len(out) == len(calls)
+        return out
+
+    return run
+
+
+def gemm(name, n, k, m):
+    return [name, [dict(n=n, k=k), PTR, PTR, m, PTR, None]]
+
+
+def least_scratch(n, k, m):
+    """T16 copy of the rows and the partials of range groups of 4, the least
+    that a product of 33 and more rows can do with."""
+    ng = -(-k // 4096)
+    return -(-m // 16) * 16 * k + (ng * m * n * 4 if ng > 1 else 0)
+
+
+@pytest.mark.parametrize("n,k", [(6400, 18944), (4032, 32768), (3584, 18944), (37888, 3584), (896, 4864),
+                                 (1536, 8960), (16, 32768), (8192, 4160)])
+def test_noalloc_takes_every_product_whose_least_scratch_fits(host, n, k):
+    """The row tile and the range groups chosen for speed must not cost a
+    product its place in the fixed scratch (6400 x 18944 at 122..127 rows and
+    4032 x 32768 at 114..127 fit only with groups of 4)."""
+    ms = list(range(33, 161)) + list(range(161, 2049, 37))
+    for m, (st, launches, alloc) in zip(ms, host([gemm("lgx_q8_gemm_noalloc", n, k, m) for m in ms])):
+        fits = least_scratch(n, k, m) <= 32 << 20
+        assert st == ("LGX_OK" if fits else "LGX_OUT_OF_BOUNDS"), (m, st)
+        assert alloc == 0 and bool(launches) == fits

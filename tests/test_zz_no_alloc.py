@@ -33,6 +33,7 @@ def _bits(t):
     (8960, 1536, (64, 1)),      # streaming, then the grouped M = 1 GEMV
     (8960, 1536, (200, 130)),   # tiled product (T16 copy; one group straight into y)
     (1536, 8960, (160, 128)),   # tiled product with group partials + combine
+    (6400, 18944, (127, 40)),   # larger range groups than lgx_q8_gemm's, to fit the scratch
 ])
 def test_noalloc_equals_q8_gemm_two_calls(ctx, orc, n, k, ms):
     t = ctx.torch
