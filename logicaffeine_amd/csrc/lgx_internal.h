@@ -688,13 +688,18 @@ inline lgx_status launch_prefill_attn(lgx_ctx* c, const lgx_attn_args& a, int d,
     const int k = prefill_attn_kernel(d, a.hq / a.hkv);
     if (k < 0) return fail(LGX_UNSUPPORTED, "prefill attention shape");
     const int qb = 32 / (a.hq / a.hkv);           // query rows per workgroup (PFA_R / heads)
-    // per chunk, the runs of LGX_PFA_SEG query blocks in eights (one per XCD)
+    // along x the runs of query blocks (LGX_PFA_SEG, or all of them where they
+    // are fewer) in eights, one per XCD; along y and z the chunks.  All of it
+    // along x, and four blocks to every run, put 4.2 million (sequence, KV
+    // head, chunk) triples of one block past the 2^32 threads of a dimension
     const int64_t nqb = (std::max(a.qpr, 1) + qb - 1) / qb;
-    const int64_t runs = (int64_t)a.B * a.hkv * ((nqb + LGX_PFA_SEG - 1) / LGX_PFA_SEG);
-    const int64_t wgs = (runs + 7) / 8 * 8 * LGX_PFA_SEG * a.ncg;
-    if (wgs > INT32_MAX) return fail(LGX_UNSUPPORTED, "prefill attention shape");
-    if (wgs == 0) return LGX_OK;
-    return launch(c, (Kern)k, dim3((unsigned)wgs), dim3(256), a, stream);
+    const int64_t seg = std::min<int64_t>(LGX_PFA_SEG, nqb);
+    const int64_t runs = (int64_t)a.B * a.hkv * ((nqb + seg - 1) / seg);
+    const int64_t wgs = (runs + 7) / 8 * 8 * seg;
+    if (wgs > UINT32_MAX / 256) return fail(LGX_UNSUPPORTED, "prefill attention shape");
+    if (wgs == 0 || a.ncg == 0) return LGX_OK;
+    return launch(c, (Kern)k, dim3((unsigned)wgs, std::min(a.ncg, LGX_PFA_Y), cdiv(a.ncg, LGX_PFA_Y)),
+                  dim3(256), a, stream);
 }
 
 }  // namespace lgxi

@@ -123,6 +123,7 @@ typedef struct {
 #define LGX_PAGE 16
 #define LGX_ATTN_CHUNK 256
 #define LGX_PFA_SEG 4          // prefill attention: query blocks of a chunk that stay on one XCD
+#define LGX_PFA_Y 32768        // prefill attention: chunks along the grid's y, the others along z
 
 // ---- decode-step glue ----
 typedef struct {

@@ -4804,18 +4804,22 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     const int qpr = max(a.qpr, 1);
     const int nqb = (qpr + QB - 1) / QB;
     // physical ids go round-robin over the 8 XCDs.  A run of PFA_SEG query
-    // blocks of one (chunk, sequence x KV head) stays on one XCD, whose L2
-    // serves their K/V; the runs of a chunk index go round the XCDs, one step
+    // blocks (or all, where there are fewer) of one (chunk, sequence x KV
+    // head) stays on one XCD, whose L2 serves their K/V; the runs of a chunk
+    // index (y and z; whole eights along x) go round the XCDs, one step
     // further with each chunk, so that sequences of different lengths (whose
     // later chunks are empty) load all XCDs alike
-    const int nseg = (nqb + PFA_SEG - 1) / PFA_SEG;
-    const int nrun = a.B * a.hkv * nseg, nrun8 = (nrun + 7) >> 3;
+    static_assert(PFA_SEG == 4, "div_seg");
+    const int seg = min(PFA_SEG, nqb);
+    auto div_seg = [&](int x) { return seg == 4 ? x >> 2 : seg == 3 ? x / 3 : x >> (seg - 1); };
+    const int nseg = div_seg(nqb + seg - 1);
+    const int nrun = a.B * a.hkv * nseg;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int ri = slot / PFA_SEG;
-    const int c = ri / nrun8;
-    const int run = 8 * (ri - c * nrun8) + ((xcd - c) & 7);
-    if (run >= nrun) return;
-    const int bg = run / nseg, qb = (run - bg * nseg) * PFA_SEG + slot % PFA_SEG;
+    const int c = blockIdx.y + blockIdx.z * LGX_PFA_Y;
+    const int ri = div_seg(slot);
+    const int run = 8 * ri + ((xcd - c) & 7);
+    if (run >= nrun || c >= a.ncg) return;
+    const int bg = run / nseg, qb = (run - bg * nseg) * seg + slot - ri * seg;
     if (qb >= nqb) return;
     const int b = bg / a.hkv, g = bg - b * a.hkv;
     const int j0 = qb * QB, t0 = c * C;

@@ -194,6 +194,20 @@ def test_prefill_attn_values_some_rows_do_not_attend_to(ctx, orc, hq, hkv, d, P)
     assert np.array_equal(out, ref, equal_nan=True)
 
 
+def test_prefill_attn_more_chunks_than_a_grid_dimension(ctx, orc):
+    """65537 chunks (a context of 16.8 million tokens on 64 pages in turn):
+    the grid's chunks continue in z."""
+    hq, hkv, d, P, ctx_len = 2, 1, 64, 2, 65536 * 256 + 38
+    rng = np.random.default_rng(5)
+    k, v, _, _ = make_cache(1, hkv, d, [64 * 16], seed=21)
+    pt = rng.integers(0, 64, (1, -(-(ctx_len + P) // 16))).astype(np.int32)
+    q = orc.gen_normal_f32(4, 31, (P, hq, d))
+    out = host(ctx.gqa_prefill_attn(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v),
+                                    ctx.to_device(pt), ctx.to_device(np.asarray([ctx_len], np.int32)),
+                                    P, ctx_len + P))
+    assert np.array_equal(out, prefill_ref(orc, q, k, v, pt, [ctx_len], P))
+
+
 def test_prefill_attn_config4_shape_sampled(ctx, orc):
     """Config-4 head layout at a 4096-token context: 64 new rows after 4032
     cached tokens (17 chunks), checked on a sample of rows."""

@@ -83,3 +83,28 @@ def test_noalloc_takes_every_product_whose_least_scratch_fits(host, n, k):
         fits = least_scratch(n, k, m) <= 32 << 20
         assert st == ("LGX_OK" if fits else "LGX_OUT_OF_BOUNDS"), (m, st)
         assert alloc == 0 and bool(launches) == fits
+
+
+def prefill(B, P, hq, hkv, d, max_seq):
+    return ["lgx_gqa_prefill_attn", [PTR] * 5 + [B, P, hq, hkv, d, -(-max_seq // 16), 1000, max_seq, PTR, None]]
+
+
+@pytest.mark.parametrize("B,P,hq,hkv,d,max_seq", [
+    (4096, 1, 8, 8, 64, 129 * 256),       # 4.2 million (sequence, KV head, chunk) triples
+    (65535, 4, 8, 1, 128, 100 * 256),
+    (1, 1, 1, 1, 64, 1 << 29),            # 2 million chunks
+    (8192, 17, 64, 8, 64, 2048),          # a run and a quarter of query blocks
+    (1, 3, 7, 1, 128, 65536 * 256),       # one chunk more than a grid's y
+    (16, 2, 28, 4, 128, 2000), (3, 33, 12, 2, 64, 100)])
+def test_prefill_attention_launches_every_block(host, B, P, hq, hkv, d, max_seq):
+    """Every (sequence, KV head, block of 32 / heads rows, chunk) has a
+    workgroup, the blocks along x in whole eights; at most 8 / 5 and 7 runs
+    more than are needed."""
+    (st, launches, _), = host([prefill(B, P, hq, hkv, d, max_seq)])
+    assert st == "LGX_OK"
+    name, gx, gy, gz, block = launches[0]
+    assert name == f"lgx_k_attn_prefill_d{d}_g{hq // hkv}" and block == 256
+    nqb, ncg = -(-P // (32 // (hq // hkv))), -(-max_seq // 256)
+    need = B * hkv * nqb
+    assert gx % 8 == 0 and need <= gx <= need * 8 / 5 + 8 * 4
+    assert ncg <= gy * gz < ncg + gy
