@@ -519,6 +519,14 @@ static lgx_status q8_gemm_impl(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
         // into y when K is one group) and the tree over the groups
         const Kern kern = tiled_kernel(c, W->n, W->k, m);
         int grp = tiled_grp(c, kern, W->n, W->k, m);
+        const int64_t slab = tiled_slab_rows((int64_t)cdiv(W->n, LGX_TG_N) * tiled_groups(W->k, grp),
+                                             tiled_rows_of(kern), m);
+        if (slab < m) {
+            for (int64_t r = 0; r < m && st == LGX_OK; r += slab)
+                st = q8_gemm_impl(c, W, xq + r * W->k, xd + r * (W->k / 32), (int)std::min(slab, m - r),
+                                  y + r * W->n, stream, scratch, cap);
+            return st;
+        }
         const size_t xbytes = ((size_t)cdiv(m, 16) * 16 * W->k + 255) / 256 * 256;
         auto bytes = [&](int g) {
             const int ng = tiled_groups(W->k, g);
@@ -608,6 +616,24 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
                         wgs += (int64_t)cdiv(W[i].n, LGX_TG_N) * cdiv(m, trows) * tiled_groups(W[i].k, grp);
                     if (wgs >= 2LL * c->ncu) break;
                 }
+            }
+        }
+        if (tiled) {
+            int64_t col_tiles = 0;
+            for (int i = 0; i < count; ++i)
+                col_tiles += (int64_t)cdiv(W[i].n, LGX_TG_N) * tiled_groups(W[i].k, grp);
+            const int64_t slab = tiled_slab_rows(col_tiles, trows, m);
+            if (slab < m) {
+                for (int64_t r = 0; r < m && st == LGX_OK; r += slab) {
+                    const float* xr[LGX_MGROUP_MAX];
+                    float* yr[LGX_MGROUP_MAX];
+                    for (int i = 0; i < count; ++i) {
+                        xr[i] = x[i] + r * W[i].k;
+                        yr[i] = y[i] + r * W[i].n;
+                    }
+                    st = lgx_q8_gemm_quantize_group(c, count, W, xr, (int)std::min(slab, m - r), yr, stream);
+                }
+                return st;
             }
         }
         // workspace: per matrix the Q8_0 activations (T16 tiles padded to 16

@@ -584,6 +584,17 @@ inline int tiled_groups(int k, int grp = LGX_TG_RANGES) { return (nranges_of(k) 
 inline int64_t tiled_grid(const lgx_gemm_tiled_args& a) {
     return ((int64_t)a.ntn * a.ntm + 7) / 8 * 8 * a.ngroups;
 }
+// Rows per call of a tiled product over `col_tiles` column tiles (of all
+// matrices and range groups): m, or equal parts of whole workgroup tiles where
+// one launch would pass 2^32 - 1 threads (outputs of 275 GB); the margin covers
+// the padding of every group to whole eights.
+inline int64_t tiled_slab_rows(int64_t col_tiles, int rows, int m) {
+    const int64_t pad = 8 * (int64_t)LGX_MGROUP_MAX * LGX_MAX_RANGES;
+    const int64_t most = std::max<int64_t>((UINT32_MAX / 256 - pad) / col_tiles, 1) * rows;
+    if (m <= most) return m;
+    const int64_t parts = (m + most - 1) / most;
+    return ((m + parts - 1) / parts + rows - 1) / rows * rows;
+}
 inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t* xt,
                                const uint16_t* xd, int m, float* part, void* stream,
                                Kern kern, int grp = LGX_TG_RANGES,

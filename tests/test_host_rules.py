@@ -108,3 +108,15 @@ def test_prefill_attention_launches_every_block(host, B, P, hq, hkv, d, max_seq)
     need = B * hkv * nqb
     assert gx % 8 == 0 and need <= gx <= need * 8 / 5 + 8 * 4
     assert ncg <= gy * gz < ncg + gy
+
+
+@pytest.mark.parametrize("n,k,m", [(16448, 64, 4194240), (16448, 64, 4194240 - 63), (128, 64, 4194240)])
+def test_products_of_the_most_rows_are_launched_whole(host, n, k, m):
+    """Products past the 2^32 threads of one launch go in several, alone and
+    in a group, and their workgroups cover every 64 x 64 tile."""
+    calls = [gemm("lgx_q8_gemm", n, k, m),
+             ["lgx_q8_gemm_quantize_group", [1, [dict(n=n, k=k)], [PTR], m, [PTR], None]]]
+    for st, launches, _ in host(calls):
+        assert st == "LGX_OK"
+        tiles = sum(gx for name, gx, *_ in launches if "gemm_tiled64" in name)
+        assert -(-n // 64) * -(-m // 64) <= tiles < -(-n // 64) * (-(-m // 64) + 2) + 16
