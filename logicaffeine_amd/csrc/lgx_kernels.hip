@@ -4749,27 +4749,36 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 //            v_mfma_f32_32x32x1 (two blocks of 32 tokens), the query rows
 //            from LDS as the A operand, block 0's values of the even and odd
 //            halves of 8 dimensions broadcast to both blocks in turn.
-//   softmax: the raw scores go through LDS; wave w takes rows 8 w ..: lane l
-//            the tokens l + 64 u, the max, p back to LDS, the halving tree
-//            (levels 128 and 64 in-lane, the rest across lanes).
+//   softmax: the raw scores go through LDS; wave w takes rows w, w + 4, ..:
+//            lane l the tokens l + 64 u, the max, p back to LDS, the halving
+//            tree (levels 128 and 64 in-lane, the rest across lanes).
 //   PV:      wave w owns dimensions [w D/4, +D/4) of all rows;
 //            v_mfma_f32_16x16x4, A = p (a lane's tokens 16 u + 4 e + g are
 //            neighbours in LDS: pfa_pos), B = V through the transposing LDS
 //            load.  V passes through two 8 KiB buffers by direct
 //            global->LDS loads, 16-byte pieces swizzled by the row.
+// Memory rounds in a row, which are what a few rows' call waits for: the page
+// entry with the length; the query rows and the K row; the first two V stages
+// during the score chain; each later one during the stage before it.  (The V
+// loads stand in inline assembly: with those it knows, the compiler moved the
+// first stage behind the score chain and waited for the next stage's before
+// reading the current one; and the query rows came in 2 or 4 rounds.)  16 x 2
+// rows at contexts up to 2000, 28/4 heads of 128: 32.6 against 35.9 us, 1 x 2
+// rows of 4/4 heads of 64 at 4000: 14.2 against 15.9.
 // 50 KiB of LDS and at most 168 VGPRs: three workgroups per compute unit,
 // whose softmax and loads overlap the others' matrix work.
 // Bound by the binary32 matrix rate (65 cycles for 2048 products; 140 us of
-// it below).  8 sequences x 128 rows at contexts up to 2000, 28/4 heads of
-// 128: 253 us, against 641 us with the chains on the VALU (8 waves, four
-// query rows, query values through scalar registers) and 387 us with each
-// XCD given whole sequences, whose lengths differ.
+// it below) and the softmax's VALU work.  8 sequences x 128 rows at contexts
+// up to 2000, 28/4 heads of 128, same inputs again and again: 209 us, 222
+// before the rounds above were taken out, 647 with the chains on the VALU (8
+// waves, four query rows, query values through scalar registers).
 // Rows of a block end at different tokens: p is 0 past a row's length, which
 // leaves o as it is unless V there is infinite or NaN; the last groups of 16
 // tokens (those that some row does not attend to in full) clear V past the
 // block's last length and, if they hold a V value that is not finite, run
-// the chain on the VALU row by row.  (o is never -0: p is 0 or above 2^-126,
-// so no product underflows to 0.)
+// the chain on the VALU row by row.  (A zero o may change its sign there: a p
+// near 2^-126 times a subnormal V can have left -0.  The merge's chain starts
+// at +0, so the sign of a zero partial is never seen.)
 // ---------------------------------------------------------------------------
 #define PFA_R 32
 #define PFA_SEG LGX_PFA_SEG
@@ -4795,8 +4804,6 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     constexpr int NC = D / 64;                    // 16-dimension column tiles per wave
     // the query rows, then (once every wave has its scores) the p rows
     __shared__ __align__(16) float p_s[PFA_R * PS];
-    // two buffers as two variables: a direct load into one is known not to
-    // alias reads of the other
     __shared__ __align__(16) uint16_t vb0[VT * D], vb1[VT * D];
     __shared__ int pg_s[C / LGX_PAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -4823,24 +4830,38 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     if (qb >= nqb) return;
     const int b = bg / a.hkv, g = bg - b * a.hkv;
     const int j0 = qb * QB, t0 = c * C;
+    // the page entry of thread t's own token, requested with the length
+    const int pge = a.page_table[(int64_t)b * a.maxp + min((t0 + tid) / LGX_PAGE, a.maxp - 1)];
     const int sl = a.seq_len[b];
     // tokens of this chunk that query row j of the sequence attends to
     auto n_of = [&](int j) { return min(C, min(max(sl + j + a.len_add, 0), a.maxlen) - t0); };
     const int nmax = n_of(min(j0 + QB, qpr) - 1);          // the block's last row
     if (nmax <= 0) return;                        // whole workgroup, before any barrier
     const int nmin = max(n_of(j0), 0);
-    if (tid < C / LGX_PAGE) {
-        int pg = 0;
-        if (tid * LGX_PAGE < nmax) pg = a.page_table[(int64_t)b * a.maxp + t0 / LGX_PAGE + tid];
-        pg_s[tid] = min(max(pg, 0), a.num_pages - 1);
-    }
-    // query rows: row r is (query row r / GQ, head r % GQ); rows past the
-    // last one repeat it and are never written out
-    for (int i = tid; i < PFA_R * D / 4; i += 256) {
-        const int r = min(i / (D / 4), QB * GQ - 1), col = (i % (D / 4)) * 4;
+    // (a page past the last length reads page 0, never used)
+    const int pgt = (tid & ~(LGX_PAGE - 1)) < nmax ? min(max(pge, 0), a.num_pages - 1) : 0;
+    if ((tid & (LGX_PAGE - 1)) == 0) pg_s[tid / LGX_PAGE] = pgt;
+    // one memory round: the query rows (row r is query row r / GQ, head r % GQ;
+    // rows past the last one repeat it and are never written out), then the
+    // thread's own K row
+    float4 q4[PFA_R * D / 1024];
+#pragma unroll
+    for (int u = 0; u < PFA_R * D / 1024; ++u) {
+        const int i = tid + 256 * u, r = min(i / (D / 4), QB * GQ - 1);
         const int jr = min(j0 + r / GQ, qpr - 1);
-        *(float4*)(p_s + (i / (D / 4)) * QS + col) =
-            *(const float4*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + col);
+        q4[u] = *(const float4*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + (i % (D / 4)) * 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint4* kr = (const uint4*)(a.kpages +
+        (((int64_t)pgt * a.hkv + g) * LGX_PAGE + (tid & (LGX_PAGE - 1))) * D);
+    uint4 kv[CPR];
+#pragma unroll
+    for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < PFA_R * D / 1024; ++u) {
+        const int i = tid + 256 * u;
+        *(float4*)(p_s + (i / (D / 4)) * QS + (i % (D / 4)) * 4) = q4[u];
     }
     __syncthreads();
 
@@ -4854,25 +4875,18 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
             const int tok = k * VT + t;
             const uint16_t* src = a.vpages +
                 (((int64_t)pg_s[tok >> 4] * a.hkv + g) * LGX_PAGE + (tok & 15)) * D + (sp ^ pfa_swz<D>(t)) * 8;
-            __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(vb + ins * 512), 16, 0, 0);
+            load_lds_16(src, (lds_void*)(vb + ins * 512));
         }
     };
 
     // ---- scores ----
     v32f s = {};
     {
-        const int tok = 64 * wave + lane;
-        const uint4* kr = (const uint4*)(a.kpages +
-            (((int64_t)pg_s[tok >> 4] * a.hkv + g) * LGX_PAGE + (tok & 15)) * D);
-        uint4 kv[CPR];
-#pragma unroll
-        for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
-        // K lands before V is requested (the compiler waits for every load in
-        // flight once direct loads are among them); V arrives meanwhile
-#pragma unroll
-        for (int j = 0; j < CPR; ++j)
-            asm volatile("" : "+v"(kv[j].x), "+v"(kv[j].y), "+v"(kv[j].z), "+v"(kv[j].w));
+        // the first two V stages arrive during the chain: their loads stand
+        // ahead of it, and the compiler does not wait for them
         stage_v(vb0, 0);
+        if (VT < nmax) stage_v(vb1, 1);
+        __builtin_amdgcn_sched_barrier(0);
         const float* qr = p_s + (lane & 31) * QS + 4 * (lane >> 5);
 #pragma unroll
         for (int j = 0; j < CPR; ++j) {
@@ -4891,7 +4905,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     }
     // lane l holds, of token 64 w + 32 blk + l % 32, the rows
     // 8 (i / 4) + 4 (l / 32) + i % 4
-    __syncthreads();                              // the query rows are fully read
+    publish_lds_loads();                          // the query rows are fully read; V stages 0 and 1 landed
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
         float* pc = p_s + 4 * (lane >> 5) * PS + pfa_pos(64 * wave + 32 * blk + (lane & 31));
@@ -4900,19 +4914,26 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     }
     __syncthreads();
 
-    // ---- softmax of rows 8 w .. 8 w + 7, four at a time ----
+    // ---- softmax: rows w, w + 4, .., four at a time (the live rows come first) ----
+    const int live = min(QB, qpr - j0) * GQ;
 #pragma unroll
-    for (int rb = 0; rb < 8; rb += 4) {
+    for (int rb = 0; rb < PFA_R; rb += 16) {
+        if (rb >= live) break;                    // uniform
         float p[4][4], mm[4], l[4];
         int nr[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = 8 * wave + rb + i, jr = j0 + r / GQ;
-            nr[i] = r < QB * GQ && jr < qpr ? n_of(jr) : 0;
+            const int r = rb + 4 * i + wave;
+            nr[i] = r < live ? n_of(j0 + r / GQ) : 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p[i][u] = p_s[r * PS + pfa_pos(lane + 64 * u)];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
             mm[i] = -__builtin_inff();
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                p[i][u] = lane + 64 * u < nr[i] ? p_s[r * PS + pfa_pos(lane + 64 * u)] * a.scale : -__builtin_inff();
+                p[i][u] = lane + 64 * u < nr[i] ? p[i][u] * a.scale : -__builtin_inff();
                 mm[i] = fmaxf(mm[i], p[i][u]);
             }
         }
@@ -4920,10 +4941,11 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
         for (int i = 0; i < 4; ++i) mm[i] = wave_max(mm[i]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = 8 * wave + rb + i;
+            const int r = rb + 4 * i + wave;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                p[i][u] = lane + 64 * u < nr[i] ? lgx_expf_nonpos(p[i][u] - mm[i]) : 0.0f;
+                const float e = lgx_expf_nonpos(p[i][u] - mm[i]);
+                p[i][u] = lane + 64 * u < nr[i] ? e : 0.0f;
                 p_s[r * PS + pfa_pos(lane + 64 * u)] = p[i][u];
             }
             l[i] = (p[i][0] + p[i][2]) + (p[i][1] + p[i][3]);   // levels 128 and 64
@@ -4933,7 +4955,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
         if (lane == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int r = 8 * wave + rb + i;
+                const int r = rb + 4 * i + wave;
                 if (nr[i] > 0) {
                     float* pp = a.part + ((((int64_t)b * qpr + j0 + r / GQ) * a.hq + g * GQ + r % GQ) * a.nchunk + c) * (D + 2);
                     pp[D] = mm[i];
@@ -4979,7 +5001,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     };
     auto pv_stage = [&](uint16_t* vb, uint16_t* vn, int k) __attribute__((always_inline)) {
         publish_lds_loads();                      // stage k landed; stage k - 1 fully read; p written
-        if ((k + 1) * VT < nmax) stage_v(vn, k + 1);
+        if (k > 0 && (k + 1) * VT < nmax) stage_v(vn, k + 1);
         const int te = min(nmax, (k + 1) * VT);
         const int tf = min(te, nmin) & ~15;       // groups before it: every row attends in full
         int ts = k * VT;

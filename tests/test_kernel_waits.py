@@ -75,3 +75,19 @@ def test_no_direct_load_is_in_flight_at_a_barrier():
     seen = kernels()
     assert any("attn_prefill_fast_d128" in k for k in seen)
     assert {k: b for k, b in ((k, unwaited_barriers(c)) for k, c in seen.items()) if b} == {}
+
+
+def test_prefill_attention_v_loads_run_under_the_matrix_chains():
+    """The exact prefill attention's V loads are in flight during products:
+    the first stages' stand ahead of the score chain, every later one's is
+    followed by products, not by a wait."""
+    seen = {k: c for k, c in kernels().items() if re.match(r"lgx_k_attn_prefill\d*_d(64|128)_g\d$", k)}
+    assert len(seen) >= 16
+    for name, code in seen.items():
+        ops = [op for _, op, _ in code]
+        loads = [i for i, op in enumerate(ops) if "load_lds" in op]
+        assert loads[0] < next(i for i, op in enumerate(ops) if op.startswith("v_mfma")), name
+        for i in loads:
+            after = next(op for op in ops[i + 1:] if op.startswith("v_mfma") or
+                         (op.startswith("s_waitcnt") and "vmcnt" in op))
+            assert after.startswith("v_mfma"), (name, i, after)
