@@ -4813,18 +4813,24 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     // physical ids go round-robin over the 8 XCDs.  A run of PFA_SEG query
     // blocks (or all, where there are fewer) of one (chunk, sequence x KV
     // head) stays on one XCD, whose L2 serves their K/V; the runs of a chunk
-    // index (y and z; whole eights along x) go round the XCDs, one step
-    // further with each chunk, so that sequences of different lengths (whose
-    // later chunks are empty) load all XCDs alike
+    // index (y and z; whole eights along x, or a.pfa_fold chunks where that
+    // many chunks' runs fit one eight) go round the XCDs, one step further with
+    // each y, so that sequences of different lengths (whose later chunks are
+    // empty) load all XCDs alike
     static_assert(PFA_SEG == 4, "div_seg");
     const int seg = min(PFA_SEG, nqb);
     auto div_seg = [&](int x) { return seg == 4 ? x >> 2 : seg == 3 ? x / 3 : x >> (seg - 1); };
     const int nseg = div_seg(nqb + seg - 1);
     const int nrun = a.B * a.hkv * nseg;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int c = blockIdx.y + blockIdx.z * LGX_PFA_Y;
+    const int slot = blockIdx.x >> 3, y = blockIdx.y + blockIdx.z * LGX_PFA_Y;
     const int ri = div_seg(slot);
-    const int run = 8 * ri + ((xcd - c) & 7);
+    int c = y, run = 8 * ri + (((blockIdx.x & 7) - y) & 7);
+    if (a.pfa_fold > 1) {                         // nrun <= 4
+        const int u = nrun == 3 ? run / 3 : run >> (nrun >> 1);
+        c = y * a.pfa_fold + u;
+        run -= u * nrun;
+        if (u >= a.pfa_fold) return;
+    }
     if (run >= nrun || c >= a.ncg) return;
     const int bg = run / nseg, qb = (run - bg * nseg) * seg + slot - ri * seg;
     if (qb >= nqb) return;

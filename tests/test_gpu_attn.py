@@ -194,10 +194,24 @@ def test_prefill_attn_values_some_rows_do_not_attend_to(ctx, orc, hq, hkv, d, P)
     assert np.array_equal(out, ref, equal_nan=True)
 
 
+@pytest.mark.parametrize("hkv,g,d,P", [(1, 7, 64, 3), (2, 2, 128, 9), (3, 1, 64, 2), (4, 6, 128, 17), (1, 8, 128, 13),
+                                       (5, 3, 64, 4), (1, 4, 64, 33)])
+def test_prefill_attn_few_runs_bit_exact(ctx, orc, hkv, g, d, P):
+    """One sequence: one to five runs of query blocks per chunk, several
+    chunks in a grid row (1, 2, 3 and 4 runs), a first and a last chunk cut."""
+    for ctx_len in (1, 250, 1500):
+        k, v, pt, maxp = make_cache(1, hkv, d, [ctx_len + P], seed=g * d + hkv + ctx_len)
+        q = orc.gen_normal_f32(6, 40 + P + ctx_len, (P, hkv * g, d))
+        out = host(ctx.gqa_prefill_attn(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v),
+                                        ctx.to_device(pt), ctx.to_device(np.asarray([ctx_len], np.int32)),
+                                        P, maxp * 16))
+        assert np.array_equal(out, prefill_ref(orc, q, k, v, pt, [ctx_len], P)), ctx_len
+
+
 def test_prefill_attn_more_chunks_than_a_grid_dimension(ctx, orc):
-    """65537 chunks (a context of 16.8 million tokens on 64 pages in turn):
-    the grid's chunks continue in z."""
-    hq, hkv, d, P, ctx_len = 2, 1, 64, 2, 65536 * 256 + 38
+    """32769 chunks of 6 KV heads (a context of 8.4 million tokens on 64 pages
+    in turn): the grid's chunks continue in z."""
+    hq, hkv, d, P, ctx_len = 6, 6, 64, 2, 32768 * 256 + 38
     rng = np.random.default_rng(5)
     k, v, _, _ = make_cache(1, hkv, d, [64 * 16], seed=21)
     pt = rng.integers(0, 64, (1, -(-(ctx_len + P) // 16))).astype(np.int32)

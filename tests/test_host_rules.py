@@ -94,20 +94,23 @@ def prefill(B, P, hq, hkv, d, max_seq):
     (65535, 4, 8, 1, 128, 100 * 256),
     (1, 1, 1, 1, 64, 1 << 29),            # 2 million chunks
     (8192, 17, 64, 8, 64, 2048),          # a run and a quarter of query blocks
-    (1, 3, 7, 1, 128, 65536 * 256),       # one chunk more than a grid's y
+    (1, 3, 7, 1, 128, 65537 * 256), (3, 3, 6, 2, 128, 32769 * 256),   # more chunks than a grid's y
     (16, 2, 28, 4, 128, 2000), (3, 33, 12, 2, 64, 100)])
 def test_prefill_attention_launches_every_block(host, B, P, hq, hkv, d, max_seq):
     """Every (sequence, KV head, block of 32 / heads rows, chunk) has a
-    workgroup, the blocks along x in whole eights; at most 8 / 5 and 7 runs
-    more than are needed."""
+    workgroup, the blocks along x in whole eights, several chunks to an eight
+    where a chunk has up to four; at most 8 / 5 and 7 runs more than are needed."""
     (st, launches, _), = host([prefill(B, P, hq, hkv, d, max_seq)])
     assert st == "LGX_OK"
     name, gx, gy, gz, block = launches[0]
     assert name == f"lgx_k_attn_prefill_d{d}_g{hq // hkv}" and block == 256
     nqb, ncg = -(-P // (32 // (hq // hkv))), -(-max_seq // 256)
     need = B * hkv * nqb
-    assert gx % 8 == 0 and need <= gx <= need * 8 / 5 + 8 * 4
-    assert ncg <= gy * gz < ncg + gy
+    assert gx % 8 == 0
+    runs = need // nqb * -(-nqb // 4)
+    fold = 8 // runs if runs <= 4 else 1
+    assert need * fold <= gx <= need * fold * 8 / 5 + 8 * 4
+    assert ncg <= gy * gz * fold < ncg + gy * fold + fold
 
 
 @pytest.mark.parametrize("n,k,m", [(16448, 64, 4194240), (16448, 64, 4194240 - 63), (128, 64, 4194240)])
