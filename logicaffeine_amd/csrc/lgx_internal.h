@@ -704,7 +704,7 @@ inline lgx_status launch_prefill_attn(lgx_ctx* c, const lgx_attn_args& a, int d,
     // along x, and four blocks to every run, put 4.2 million (sequence, KV
     // head, chunk) triples of one block past the 2^32 threads of a dimension.
     // Up to four runs share their eight with other chunks' (1 x 16 rows at a
-    // 4000-token context, 14/2 heads of 64: 19.3 against 22.9 us)
+    // 4000-token context, 14/2 heads of 64: 17.3 against 23.0 us)
     const int64_t nqb = (std::max(a.qpr, 1) + qb - 1) / qb;
     const int64_t seg = std::min<int64_t>(LGX_PFA_SEG, nqb);
     const int64_t runs = (int64_t)a.B * a.hkv * ((nqb + seg - 1) / seg);

@@ -4763,7 +4763,7 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // loads stand in inline assembly: with those it knows, the compiler moved the
 // first stage behind the score chain and waited for the next stage's before
 // reading the current one; and the query rows came in 2 or 4 rounds.)  16 x 2
-// rows at contexts up to 2000, 28/4 heads of 128: 32.6 against 35.9 us, 1 x 2
+// rows at contexts up to 2000, 28/4 heads of 128: 32 against 35.9 us, 1 x 2
 // rows of 4/4 heads of 64 at 4000: 14.2 against 15.9.
 // 50 KiB of LDS and at most 168 VGPRs: three workgroups per compute unit,
 // whose softmax and loads overlap the others' matrix work.
@@ -4850,13 +4850,12 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     // one memory round: the query rows (row r is query row r / GQ, head r % GQ;
     // rows past the last one repeat it and are never written out), then the
     // thread's own K row
-    float4 q4[PFA_R * D / 1024];
-#pragma unroll
-    for (int u = 0; u < PFA_R * D / 1024; ++u) {
-        const int i = tid + 256 * u, r = min(i / (D / 4), QB * GQ - 1);
+    v4f q4[PFA_R * D / 1024];
+    static_for<0, PFA_R * D / 1024>([&](auto U) {
+        const int i = tid + 256 * U.value, r = min(i / (D / 4), QB * GQ - 1);
         const int jr = min(j0 + r / GQ, qpr - 1);
-        q4[u] = *(const float4*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + (i % (D / 4)) * 4);
-    }
+        q4[U.value] = *(const v4f*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + (i % (D / 4)) * 4);
+    });
     __builtin_amdgcn_sched_barrier(0);
     const uint4* kr = (const uint4*)(a.kpages +
         (((int64_t)pgt * a.hkv + g) * LGX_PAGE + (tid & (LGX_PAGE - 1))) * D);
@@ -4864,11 +4863,10 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
 #pragma unroll
     for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < PFA_R * D / 1024; ++u) {
-        const int i = tid + 256 * u;
-        *(float4*)(p_s + (i / (D / 4)) * QS + (i % (D / 4)) * 4) = q4[u];
-    }
+    static_for<0, PFA_R * D / 1024>([&](auto U) {
+        const int i = tid + 256 * U.value;
+        *(v4f*)(p_s + (i / (D / 4)) * QS + (i % (D / 4)) * 4) = q4[U.value];
+    });
     __syncthreads();
 
     // direct loads of V tokens [VT k, +VT) of the chunk: 8 wave instructions

@@ -88,6 +88,24 @@ def test_prefill_attention_v_loads_run_under_the_matrix_chains():
         loads = [i for i, op in enumerate(ops) if "load_lds" in op]
         assert loads[0] < next(i for i, op in enumerate(ops) if op.startswith("v_mfma")), name
         for i in loads:
-            after = next(op for op in ops[i + 1:] if op.startswith("v_mfma") or
-                         (op.startswith("s_waitcnt") and "vmcnt" in op))
-            assert after.startswith("v_mfma"), (name, i, after)
+            state = 0                 # memory operations since the load
+            for op in ops[i + 1:]:
+                if op.startswith("v_mfma"):
+                    break
+                if re.match(r"(global|buffer|flat|scratch)_(load|store|atomic)", op):
+                    state += 1
+                wait = re.search(r"vmcnt\((\d+)\)", op)
+                assert not (wait and state >= int(wait.group(1))), (name, i, op)
+
+
+def test_kernels_keep_their_arrays_in_registers():
+    """No kernel spills or indexes an array in scratch memory, except the two
+    largest fast prefill attention forms (20 bytes, at 128 registers)."""
+    if not os.path.exists(lgx.HSACO_PATH):
+        pytest.skip("no built code object")
+    readelf = os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf")
+    notes = subprocess.run([readelf, "--notes", lgx.HSACO_PATH], check=True, capture_output=True, text=True).stdout
+    size = dict(re.findall(r"\.name: +(lgx_k_\w+)\n\s+\.private_segment_fixed_size: (\d+)", notes))
+    assert len(size) > 100
+    kept = {f"lgx_k_attn_prefill_fast_d128_g{g}" for g in (7, 8)}
+    assert {k: int(v) for k, v in size.items() if int(v) > (20 if k in kept else 0)} == {}
