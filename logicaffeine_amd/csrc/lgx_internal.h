@@ -142,7 +142,9 @@ enum Kern {
     K_GEMM_TILED32,
     K_PFA_D64_G1,    // + (gq - 1)
     K_PFA_D128_G1 = K_PFA_D64_G1 + 8,
-    K_SAMPLE_PARTIAL = K_PFA_D128_G1 + 8,
+    K_PFA16_D64_G1 = K_PFA_D128_G1 + 8,
+    K_PFA16_D128_G1 = K_PFA16_D64_G1 + 8,
+    K_SAMPLE_PARTIAL = K_PFA16_D128_G1 + 8,
     K_SAMPLE_FINAL,
     K_GEMM_MFMA16_QKV,
     K_GEMM_MFMA16_SWIGLU,
@@ -196,6 +198,10 @@ inline const char* const kKernelNames[] = {
     "lgx_k_attn_prefill_d128_g1", "lgx_k_attn_prefill_d128_g2", "lgx_k_attn_prefill_d128_g3",
     "lgx_k_attn_prefill_d128_g4", "lgx_k_attn_prefill_d128_g5", "lgx_k_attn_prefill_d128_g6",
     "lgx_k_attn_prefill_d128_g7", "lgx_k_attn_prefill_d128_g8",
+    "lgx_k_attn_prefill16_d64_g1", "lgx_k_attn_prefill16_d64_g2", "lgx_k_attn_prefill16_d64_g3", "lgx_k_attn_prefill16_d64_g4",
+    "lgx_k_attn_prefill16_d64_g5", "lgx_k_attn_prefill16_d64_g6", "lgx_k_attn_prefill16_d64_g7", "lgx_k_attn_prefill16_d64_g8",
+    "lgx_k_attn_prefill16_d128_g1", "lgx_k_attn_prefill16_d128_g2", "lgx_k_attn_prefill16_d128_g3", "lgx_k_attn_prefill16_d128_g4",
+    "lgx_k_attn_prefill16_d128_g5", "lgx_k_attn_prefill16_d128_g6", "lgx_k_attn_prefill16_d128_g7", "lgx_k_attn_prefill16_d128_g8",
     "lgx_k_sample_partial", "lgx_k_sample_final",
     "lgx_k_q8_gemm_mfma16_qkv", "lgx_k_q8_gemm_mfma16_swiglu", "lgx_k_add_rmsnorm_quant_w",
     "lgx_k_q8_gemm_mfma16_group", "lgx_k_q8_gemm_tiled64_group",
@@ -223,8 +229,10 @@ inline int attn_kernel(int d, int gq) {
 }
 
 // Prefill (multi-query causal) attention kernel for head_dim d, gq heads per KV head.
-inline int prefill_attn_kernel(int d, int gq) {
+// The kernel with `rows` = 32 or 16 (query row, head) pairs per workgroup.
+inline int prefill_attn_kernel(int d, int gq, int rows = 32) {
     if (gq < 1 || gq > 8) return -1;
+    if (rows == 16) return (d == 64 ? K_PFA16_D64_G1 : K_PFA16_D128_G1) + gq - 1;
     return (d == 64 ? K_PFA_D64_G1 : K_PFA_D128_G1) + gq - 1;
 }
 // Debug/tuning knobs read once per ctx from the environment:
@@ -263,6 +271,7 @@ struct lgx_ctx {
     int norm_waves = 1;           // LGX_NORM_WAVES: rows (waves) per workgroup of the wave norm (0: off)
     bool lm_cert = true;          // LGX_LM_CERT=0: greedy tied lm_head through the full logits
     bool tiled_s4 = true;         // LGX_TILED_S4=0: tiled products always in stages of 2 pairs
+    int pfa_rows = 0;             // LGX_PFA_ROWS: force 32 / 16 (query row, head) pairs per prefill attention workgroup
     bool prefill_serial = false;  // LGX_PREFILL=serial: prefill as P decode passes
     int prefill_chunk = 0;        // LGX_PREFILL_CHUNK: positions per prefill chunk (0: by batch)
     int ncu = 256;                // compute units of the device
@@ -692,13 +701,35 @@ inline lgx_status launch_prefill_attn_fast(lgx_ctx* c, const lgx_attn_args& a, i
     if (wgs == 0) return LGX_OK;
     return launch(c, (Kern)k, dim3((unsigned)wgs), dim3(64 * gq), a, stream);
 }
+// (query row, head) pairs per workgroup of the prefill attention: 32, or 16
+// (half the matrix time per workgroup, K and V converted for half the rows)
+// where the larger blocks leave the device idle or half empty.  w: workgroups
+// at full lengths.  Measured over every heads-per-group at 1 to 256 rows, 1 to
+// 16 sequences, contexts 64 to 4000 (16 against 32, us):
+//  - up to one and a half workgroups of 16 per compute unit: 0.67-0.80 of the
+//    time (1 x 16 rows at 4000 tokens, 4/4 heads of 64: 11.6 against 14.7);
+//  - up to three of 32 and no more slots in all: 0.75-1.03 (16 x 8 rows at 2000,
+//    14/2 heads of 64: 0.95; beyond, 16 x 16, 20/4 of 128: 1.03);
+//  - at most 0.8 of the slots: 0.5-0.95 (16 x 2 rows at 2000, 4/4 heads of 64:
+//    14.4 against 19.5); with 0.83 of them (16 x 13, 20/4 of 128) 1.15.
+// LGX_PFA_ROWS forces one.
+inline int prefill_attn_rows(const lgx_ctx* c, const lgx_attn_args& a) {
+    if (c->pfa_rows == 16 || c->pfa_rows == 32) return c->pfa_rows;
+    const int gq = a.hq / a.hkv, q = std::max(a.qpr, 1);
+    const int64_t n32 = cdiv(q, 32 / gq), n16 = cdiv(q, 16 / gq);
+    const int64_t per = (int64_t)a.B * a.hkv * a.ncg;
+    if (2 * per * n16 <= 3LL * c->ncu) return 16;
+    if (n16 <= 2 * n32 && per * n32 <= 3LL * c->ncu) return 16;
+    // (the last bound keeps the longer grids of 16 within a launch)
+    return 5 * n16 <= 8 * n32 && (int64_t)a.B * a.hkv * n32 <= 1 << 20 ? 16 : 32;
+}
 // Launch of the prefill attention over B sequences x a.qpr query rows: one
-// workgroup per (sequence, KV head, chunk of the grid, block of 32 / heads
-// query rows).
+// workgroup per (sequence, KV head, chunk of the grid, block of 32 / heads or
+// 16 / heads query rows).
 inline lgx_status launch_prefill_attn(lgx_ctx* c, const lgx_attn_args& a, int d, void* stream) {
-    const int k = prefill_attn_kernel(d, a.hq / a.hkv);
+    const int gq = a.hq / a.hkv, rows = prefill_attn_rows(c, a), qb = rows / gq;   // qb query rows per workgroup
+    const int k = prefill_attn_kernel(d, gq, rows);
     if (k < 0) return fail(LGX_UNSUPPORTED, "prefill attention shape");
-    const int qb = 32 / (a.hq / a.hkv);           // query rows per workgroup (PFA_R / heads)
     // along x the runs of query blocks (LGX_PFA_SEG, or all of them where they
     // are fewer) in eights, one per XCD; along y and z the chunks.  All of it
     // along x, and four blocks to every run, put 4.2 million (sequence, KV
@@ -713,8 +744,8 @@ inline lgx_status launch_prefill_attn(lgx_ctx* c, const lgx_attn_args& a, int d,
     if (wgs == 0 || a.ncg == 0) return LGX_OK;
     lgx_attn_args p = a;
     p.pfa_fold = runs <= 4 ? 8 / (int)runs : 1;
-    const int rows = (int)cdiv(a.ncg, p.pfa_fold);
-    return launch(c, (Kern)k, dim3((unsigned)wgs, std::min(rows, LGX_PFA_Y), cdiv(rows, LGX_PFA_Y)),
+    const int ys = (int)cdiv(a.ncg, p.pfa_fold);
+    return launch(c, (Kern)k, dim3((unsigned)wgs, std::min(ys, LGX_PFA_Y), cdiv(ys, LGX_PFA_Y)),
                   dim3(256), p, stream);
 }
 

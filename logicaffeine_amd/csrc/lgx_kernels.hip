@@ -4742,13 +4742,15 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // fmaf of 64 lanes but takes 32 rows against one converted K or V value, so
 // the conversions, the LDS reads and the query broadcasts are shared by all
 // rows.
-// Workgroup: 4 waves for (sequence b, KV head g, PFA_QB query rows, chunk c);
-// the (query row, head) pairs of the group, row-major, are the PFA_R = 32
-// rows of the products.
-//   scores:  wave w owns tokens 64 w + lane (the lane's K row in registers);
-//            v_mfma_f32_32x32x1 (two blocks of 32 tokens), the query rows
-//            from LDS as the A operand, block 0's values of the even and odd
-//            halves of 8 dimensions broadcast to both blocks in turn.
+// Workgroup: 4 waves for (sequence b, KV head g, QB = R / GQ query rows, chunk
+// c); the (query row, head) pairs of the group, row-major, are the R = 32 or
+// 16 rows of the products (prefill_attn_rows has the rule).
+//   scores:  wave w owns tokens 64 w + lane (the lane's K row in registers),
+//            the query rows from LDS as the A operand.  R = 32:
+//            v_mfma_f32_32x32x1 (two blocks of 32 tokens), block 0's values of
+//            the even and odd halves of 8 dimensions broadcast to both blocks
+//            in turn.  R = 16: v_mfma_f32_16x16x1 (four blocks of 16 tokens),
+//            block b's values the dimensions 4 b .. + 3 of 16, broadcast in turn.
 //   softmax: the raw scores go through LDS; wave w takes rows w, w + 4, ..:
 //            lane l the tokens l + 64 u, the max, p back to LDS, the halving
 //            tree (levels 128 and 64 in-lane, the rest across lanes).
@@ -4763,15 +4765,15 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // loads stand in inline assembly: with those it knows, the compiler moved the
 // first stage behind the score chain and waited for the next stage's before
 // reading the current one; and the query rows came in 2 or 4 rounds.)  16 x 2
-// rows at contexts up to 2000, 28/4 heads of 128: 32 against 35.9 us, 1 x 2
-// rows of 4/4 heads of 64 at 4000: 14.2 against 15.9.
-// 50 KiB of LDS and at most 168 VGPRs: three workgroups per compute unit,
-// whose softmax and loads overlap the others' matrix work.
+// rows at contexts up to 2000, 28/4 heads of 128: 32 us against 35.9 with R =
+// 32, 23.2 with R = 16 (41.5 with the chains on the VALU: 8 waves, four query
+// rows, query values through scalar registers).
+// 50 or 33 KiB of LDS and at most 168 or 128 VGPRs: three or four workgroups
+// per compute unit, whose softmax and loads overlap the others' matrix work.
 // Bound by the binary32 matrix rate (65 cycles for 2048 products; 140 us of
 // it below) and the softmax's VALU work.  8 sequences x 128 rows at contexts
-// up to 2000, 28/4 heads of 128, same inputs again and again: 209 us, 222
-// before the rounds above were taken out, 647 with the chains on the VALU (8
-// waves, four query rows, query values through scalar registers).
+// up to 2000, 28/4 heads of 128, same inputs again and again: 205 us, 222
+// before the rounds above were taken out, 647 on the VALU.
 // Rows of a block end at different tokens: p is 0 past a row's length, which
 // leaves o as it is unless V there is infinite or NaN; the last groups of 16
 // tokens (those that some row does not attend to in full) clear V past the
@@ -4780,7 +4782,6 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // near 2^-126 times a subnormal V can have left -0.  The merge's chain starts
 // at +0, so the sign of a zero partial is never seen.)
 // ---------------------------------------------------------------------------
-#define PFA_R 32
 #define PFA_SEG LGX_PFA_SEG
 
 // Column of token t in a p row: the tokens 16 u + 4 e + g, e = 0..3, of one
@@ -4794,16 +4795,17 @@ __device__ __forceinline__ int pfa_swz(int t) {
     return D == 128 ? (t & 7) << 1 : ((t >> 1) & 3) << 1;
 }
 
-template <int D, int GQ>
+template <int D, int GQ, int R>
 __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     constexpr int C = LGX_ATTN_CHUNK;
-    constexpr int QB = PFA_R / GQ;                // query rows of the workgroup
+    constexpr int QB = R / GQ;                    // query rows of the workgroup
+    constexpr int RT = R / 16;                    // row tiles of the PV products
     constexpr int CPR = D / 8;                    // 16-byte pieces per row
     constexpr int QS = D + 4, PS = C + 8;         // row strides in floats
     constexpr int VT = 8192 / (2 * D);            // tokens per V buffer
     constexpr int NC = D / 64;                    // 16-dimension column tiles per wave
     // the query rows, then (once every wave has its scores) the p rows
-    __shared__ __align__(16) float p_s[PFA_R * PS];
+    __shared__ __align__(16) float p_s[R * PS];
     __shared__ __align__(16) uint16_t vb0[VT * D], vb1[VT * D];
     __shared__ int pg_s[C / LGX_PAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -4850,8 +4852,8 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     // one memory round: the query rows (row r is query row r / GQ, head r % GQ;
     // rows past the last one repeat it and are never written out), then the
     // thread's own K row
-    v4f q4[PFA_R * D / 1024];
-    static_for<0, PFA_R * D / 1024>([&](auto U) {
+    v4f q4[R * D / 1024];
+    static_for<0, R * D / 1024>([&](auto U) {
         const int i = tid + 256 * U.value, r = min(i / (D / 4), QB * GQ - 1);
         const int jr = min(j0 + r / GQ, qpr - 1);
         q4[U.value] = *(const v4f*)(a.q + (((int64_t)b * qpr + jr) * a.hq + g * GQ + r % GQ) * D + (i % (D / 4)) * 4);
@@ -4863,7 +4865,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
 #pragma unroll
     for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
     __builtin_amdgcn_sched_barrier(0);
-    static_for<0, PFA_R * D / 1024>([&](auto U) {
+    static_for<0, R * D / 1024>([&](auto U) {
         const int i = tid + 256 * U.value;
         *(v4f*)(p_s + (i / (D / 4)) * QS + (i % (D / 4)) * 4) = q4[U.value];
     });
@@ -4884,44 +4886,64 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     };
 
     // ---- scores ----
-    v32f s = {};
-    {
-        // the first two V stages arrive during the chain: their loads stand
-        // ahead of it, and the compiler does not wait for them
-        stage_v(vb0, 0);
-        if (VT < nmax) stage_v(vb1, 1);
-        __builtin_amdgcn_sched_barrier(0);
+    // the first two V stages arrive during the chain: their loads stand ahead
+    // of it, and the compiler does not wait for them
+    stage_v(vb0, 0);
+    if (VT < nmax) stage_v(vb1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    auto kval = [&](auto DIM) {                   // dimension DIM of the lane's K row
+        constexpr int j = DIM.value >> 3, e = DIM.value & 7;
+        const uint32_t w4[4] = {kv[j].x, kv[j].y, kv[j].z, kv[j].w};
+        return h2f(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu);
+    };
+    if constexpr (R == 32) {
+        v32f s = {};
         const float* qr = p_s + (lane & 31) * QS + 4 * (lane >> 5);
+        static_for<0, CPR>([&](auto J) {
+            const float4 qv = *(const float4*)(qr + 8 * J.value);
+            const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
+            static_for<0, 4>([&](auto E) {
+                s = __builtin_amdgcn_mfma_f32_32x32x1f32(qa[E.value], kval(IdxC<8 * J.value + E.value>{}), s, 1, 0, 0);
+            });
+            static_for<0, 4>([&](auto E) {
+                s = __builtin_amdgcn_mfma_f32_32x32x1f32(qa[E.value], kval(IdxC<8 * J.value + 4 + E.value>{}), s, 1, 1, 0);
+            });
+        });
+        // lane l holds, of token 64 w + 32 blk + l % 32, the rows
+        // 8 (i / 4) + 4 (l / 32) + i % 4
+        publish_lds_loads();                      // the query rows are fully read; V stages 0 and 1 landed
 #pragma unroll
-        for (int j = 0; j < CPR; ++j) {
-            const float4 q4 = *(const float4*)(qr + 8 * j);
-            const uint32_t w4[4] = {kv[j].x, kv[j].y, kv[j].z, kv[j].w};
-            const float qa[4] = {q4.x, q4.y, q4.z, q4.w};
+        for (int blk = 0; blk < 2; ++blk) {
+            float* pc = p_s + 4 * (lane >> 5) * PS + pfa_pos(64 * wave + 32 * blk + (lane & 31));
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                s = __builtin_amdgcn_mfma_f32_32x32x1f32(
-                    qa[e], h2f(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu), s, 1, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                s = __builtin_amdgcn_mfma_f32_32x32x1f32(
-                    qa[e], h2f(e & 1 ? w4[2 + (e >> 1)] >> 16 : w4[2 + (e >> 1)] & 0xffffu), s, 1, 1, 0);
+            for (int i = 0; i < 16; ++i) pc[(8 * (i >> 2) + (i & 3)) * PS] = s[16 * blk + i];
         }
-    }
-    // lane l holds, of token 64 w + 32 blk + l % 32, the rows
-    // 8 (i / 4) + 4 (l / 32) + i % 4
-    publish_lds_loads();                          // the query rows are fully read; V stages 0 and 1 landed
+    } else {
+        v16f s = {};
+        const float* qr = p_s + (lane & 15) * QS + 4 * (lane >> 4);
+        static_for<0, D / 16>([&](auto J) {
+            const float4 qv = *(const float4*)(qr + 16 * J.value);
+            const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
+            static_for<0, 16>([&](auto E) {
+                constexpr int e = E.value;
+                s = __builtin_amdgcn_mfma_f32_16x16x1f32(qa[e & 3], kval(IdxC<16 * J.value + e>{}), s, 2, e >> 2, 0);
+            });
+        });
+        // lane l holds, of token 64 w + 16 blk + l % 16, the rows 4 (l / 16) + i
+        publish_lds_loads();                      // as above
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-        float* pc = p_s + 4 * (lane >> 5) * PS + pfa_pos(64 * wave + 32 * blk + (lane & 31));
+        for (int blk = 0; blk < 4; ++blk) {
+            float* pc = p_s + 4 * (lane >> 4) * PS + pfa_pos(64 * wave + 16 * blk + (lane & 15));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) pc[(8 * (i >> 2) + (i & 3)) * PS] = s[16 * blk + i];
+            for (int i = 0; i < 4; ++i) pc[i * PS] = s[4 * blk + i];
+        }
     }
     __syncthreads();
 
     // ---- softmax: rows w, w + 4, .., four at a time (the live rows come first) ----
     const int live = min(QB, qpr - j0) * GQ;
 #pragma unroll
-    for (int rb = 0; rb < PFA_R; rb += 16) {
+    for (int rb = 0; rb < R; rb += 16) {
         if (rb >= live) break;                    // uniform
         float p[4][4], mm[4], l[4];
         int nr[4];
@@ -4971,14 +4993,14 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
 
     // ---- PV ----
     const int qc = lane & 15, kg = lane >> 4;
-    v4f o[2][NC];
+    v4f o[RT][NC];
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < NC; ++ct) o[rt][ct] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    auto pv_load = [&](uint16_t* vb, int ts, int k, float4 (&pa)[2], float (&vf)[NC][4]) __attribute__((always_inline)) {
+    auto pv_load = [&](uint16_t* vb, int ts, int k, float4 (&pa)[RT], float (&vf)[NC][4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) pa[rt] = *(const float4*)(p_s + (16 * rt + qc) * PS + ts + 4 * kg);
+        for (int rt = 0; rt < RT; ++rt) pa[rt] = *(const float4*)(p_s + (16 * rt + qc) * PS + ts + 4 * kg);
         // lane (qc, kg) loads token ts + 4 (qc / 4) + kg, dimensions
         // 4 (qc % 4) .. of the column tile, and receives dimension qc of the
         // tokens ts + 4 e + kg
@@ -4992,13 +5014,13 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
             for (int e = 0; e < 4; ++e) vf[ct][e] = h2f((uint16_t)vw[e]);
         }
     };
-    auto pv_mul = [&](const float4 (&pa)[2], const float (&vf)[NC][4]) __attribute__((always_inline)) {
+    auto pv_mul = [&](const float4 (&pa)[RT], const float (&vf)[NC][4]) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
+                for (int rt = 0; rt < RT; ++rt) {
                     const float pe = e == 0 ? pa[rt].x : e == 1 ? pa[rt].y : e == 2 ? pa[rt].z : pa[rt].w;
                     o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(pe, vf[ct][e], o[rt][ct], 0, 0, 0);
                 }
@@ -5010,13 +5032,13 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
         const int tf = min(te, nmin) & ~15;       // groups before it: every row attends in full
         int ts = k * VT;
         for (; ts < tf; ts += 16) {
-            float4 pa[2];
+            float4 pa[RT];
             float vf[NC][4];
             pv_load(vb, ts, k, pa, vf);
             pv_mul(pa, vf);
         }
         for (; ts < te; ts += 16) {               // a row ends in here
-            float4 pa[2];
+            float4 pa[RT];
             float vf[NC][4];
             pv_load(vb, ts, k, pa, vf);
             bool bad = false;
@@ -5038,7 +5060,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
                     const int col = 16 * (wave * NC + ct) + qc;
                     const float v = h2f(vb[tr * D + ((col >> 3) ^ pfa_swz<D>(tr)) * 8 + (col & 7)]);
 #pragma unroll
-                    for (int rt = 0; rt < 2; ++rt)
+                    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int r = 16 * rt + 4 * kg + i;
@@ -5055,7 +5077,7 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
         if ((k + 1) * VT < nmax) pv_stage(vb1, vb0, k + 1);
     }
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int r = 16 * rt + 4 * kg + i, jr = j0 + r / GQ;
@@ -5069,8 +5091,12 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
 
 #define LGX_PFA_KERNELS(D, G)                                                                     \
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))        \
-    void lgx_k_attn_prefill_d##D##_g##G(const lgx_attn_args a) {                                                                 \
-        attn_prefill_body<D, G>(a);                                                              \
+    void lgx_k_attn_prefill_d##D##_g##G(const lgx_attn_args a) {                                \
+        attn_prefill_body<D, G, 32>(a);                                                          \
+    }                                                                                            \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))        \
+    void lgx_k_attn_prefill16_d##D##_g##G(const lgx_attn_args a) {                              \
+        attn_prefill_body<D, G, 16>(a);                                                          \
     }
 LGX_PFA_KERNELS(64, 1)
 LGX_PFA_KERNELS(64, 2)

@@ -194,6 +194,28 @@ def test_prefill_attn_values_some_rows_do_not_attend_to(ctx, orc, hq, hkv, d, P)
     assert np.array_equal(out, ref, equal_nan=True)
 
 
+@pytest.mark.parametrize("rows", [16, 32])
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_attn_both_block_sizes_bit_exact(monkeypatch, orc, rows, d):
+    """16 and 32 (query row, head) pairs per workgroup, every head group: one
+    block exactly full, one row more, a block cut by the chunk's end, NaN in a
+    V row that only the last query rows attend to."""
+    monkeypatch.setenv("LGX_PFA_ROWS", str(rows))
+    c = lgx.Context(0)
+    try:
+        for g in range(1, 9):
+            for P in (rows // g, rows // g + 1, 2 * (rows // g) + 1):
+                ctx_len = [0, 256 - P // 2, 700]
+                k, v, pt, maxp = make_cache(3, 2, d, [n + P for n in ctx_len], seed=g * d + P)
+                v[pt[1, (255 + P // 2) // 16], :, (255 + P // 2) % 16, 1::5] = 0x7E00
+                q = orc.gen_normal_f32(7, g + d + P, (3 * P, 2 * g, d))
+                out = host(c.gqa_prefill_attn(c.to_device(q), c.to_device(k), c.to_device(v), c.to_device(pt),
+                                              c.to_device(np.asarray(ctx_len, np.int32)), P, maxp * 16))
+                assert np.array_equal(out, prefill_ref(orc, q, k, v, pt, ctx_len, P), equal_nan=True), (g, P)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("hkv,g,d,P", [(1, 7, 64, 3), (2, 2, 128, 9), (3, 1, 64, 2), (4, 6, 128, 17), (1, 8, 128, 13),
                                        (5, 3, 64, 4), (1, 4, 64, 33)])
 def test_prefill_attn_few_runs_bit_exact(ctx, orc, hkv, g, d, P):
@@ -211,7 +233,7 @@ def test_prefill_attn_few_runs_bit_exact(ctx, orc, hkv, g, d, P):
 def test_prefill_attn_more_chunks_than_a_grid_dimension(ctx, orc):
     """32769 chunks of 6 KV heads (a context of 8.4 million tokens on 64 pages
     in turn): the grid's chunks continue in z."""
-    hq, hkv, d, P, ctx_len = 6, 6, 64, 2, 32768 * 256 + 38
+    hq, hkv, d, P, ctx_len = 6, 6, 64, 2, 32768 * 256 + 38    # runs of one block: fold 1
     rng = np.random.default_rng(5)
     k, v, _, _ = make_cache(1, hkv, d, [64 * 16], seed=21)
     pt = rng.integers(0, 64, (1, -(-(ctx_len + P) // 16))).astype(np.int32)

@@ -94,17 +94,18 @@ def prefill(B, P, hq, hkv, d, max_seq):
     (65535, 4, 8, 1, 128, 100 * 256),
     (1, 1, 1, 1, 64, 1 << 29),            # 2 million chunks
     (8192, 17, 64, 8, 64, 2048),          # a run and a quarter of query blocks
-    (1, 3, 7, 1, 128, 65537 * 256), (3, 3, 6, 2, 128, 32769 * 256),   # more chunks than a grid's y
+    (1, 3, 7, 1, 128, 65537 * 256), (3, 3, 12, 2, 128, 32769 * 256),  # more chunks than a grid's y
     (16, 2, 28, 4, 128, 2000), (3, 33, 12, 2, 64, 100)])
 def test_prefill_attention_launches_every_block(host, B, P, hq, hkv, d, max_seq):
-    """Every (sequence, KV head, block of 32 / heads rows, chunk) has a
+    """Every (sequence, KV head, block of 32 / heads or 16 / heads rows, chunk) has a
     workgroup, the blocks along x in whole eights, several chunks to an eight
     where a chunk has up to four; at most 8 / 5 and 7 runs more than are needed."""
     (st, launches, _), = host([prefill(B, P, hq, hkv, d, max_seq)])
     assert st == "LGX_OK"
     name, gx, gy, gz, block = launches[0]
-    assert name == f"lgx_k_attn_prefill_d{d}_g{hq // hkv}" and block == 256
-    nqb, ncg = -(-P // (32 // (hq // hkv))), -(-max_seq // 256)
+    rows = 16 if name.startswith("lgx_k_attn_prefill16") else 32
+    assert name == f"lgx_k_attn_prefill{'16' if rows == 16 else ''}_d{d}_g{hq // hkv}" and block == 256
+    nqb, ncg = -(-P // (rows // (hq // hkv))), -(-max_seq // 256)
     need = B * hkv * nqb
     assert gx % 8 == 0
     runs = need // nqb * -(-nqb // 4)
