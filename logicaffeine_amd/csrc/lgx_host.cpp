@@ -701,6 +701,7 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
                 a.ngroups = tiled_groups(W[i].k, grp);
                 a.ntn = (int)cdiv(W[i].n, LGX_TG_N);
                 a.ntm = (int)cdiv(m, trows);
+                a.whole = tiled_whole(c, a, trows);
                 const int64_t end = ta.wg0[i] + tiled_grid(a);
                 if (end > INT32_MAX) return fail(LGX_OUT_OF_BOUNDS, "grouped product too large");
                 ta.wg0[i + 1] = (int32_t)end;

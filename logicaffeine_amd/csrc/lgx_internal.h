@@ -589,9 +589,27 @@ inline lgx_status run_q8(lgx_ctx* c, Kern kern, const lgx_q8_matrix* W, const fl
 // sq (T16) / sd instead of part.
 inline int tiled_rows_of(Kern kern) { return kern == K_GEMM_TILED64 ? 64 : 32; }
 inline int tiled_groups(int k, int grp = LGX_TG_RANGES) { return (nranges_of(k) + grp - 1) / grp; }
-// Grid of the tiled product: each group's tiles in whole eights (one per XCD).
+// Grid of the tiled product: the tiles of all groups, or each group's, in
+// whole eights (one per XCD).
 inline int64_t tiled_grid(const lgx_gemm_tiled_args& a) {
-    return ((int64_t)a.ntn * a.ntm + 7) / 8 * 8 * a.ngroups;
+    const int64_t per_g = (int64_t)a.ntn * a.ntm;
+    return a.whole ? (per_g * a.ngroups + 7) / 8 * 8 : (per_g + 7) / 8 * 8 * a.ngroups;
+}
+// Order of the tiles of a product over the XCDs: whole runs of all groups'
+// tiles, so that a group's activations are read by one or two XCDs, or a share
+// of every group's, so that each XCD has the same part of a short last group.
+// Runs where the last group lacks nothing (512 x 32768, 32 groups, us at 33 /
+// 64 / 192 rows: 14.2 / 15.3 / 26.6 against 15.3 / 17.0 / 29.0; 8192 x 4096
+// alike), where a compute unit has one workgroup at most and so no tail (896 x
+// 4864 at 33 to 96 rows, 1536 x 1536 at 33 to 160: 0.93-0.99), and where
+// little is missing from a small grid (1536 x 8960 at 33 to 96 rows, 8 blocks
+// of 288 missing, 432 to 648 workgroups: 0.96-0.99); else shares (2048 x 1536
+// at 160 rows, a quarter missing: 11.7 against 13.1; 3584 x 18944 at 2047
+// rows, 5 groups of 4.6: 0.94-0.96).
+inline int tiled_whole(const lgx_ctx* c, const lgx_gemm_tiled_args& a, int rows) {
+    const int64_t wgs = (int64_t)a.ntn * a.ntm * a.ngroups;
+    const int all = a.ngroups * a.grp * LGX_Q8_RANGE_BLOCKS, miss = all - (a.k >> 5);
+    return miss == 0 || wgs <= c->ncu || (32 * miss <= all && wgs * rows <= 96LL * c->ncu);
 }
 // Rows per call of a tiled product over `col_tiles` column tiles (of all
 // matrices and range groups): m, or equal parts of whole workgroup tiles where
@@ -630,6 +648,7 @@ inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
     }
     a.ntn = (int)cdiv(W->n, LGX_TG_N);
     a.ntm = (int)cdiv(m, mrows);
+    a.whole = tiled_whole(c, a, mrows);
     const int64_t wgs = (int64_t)a.ntn * a.ntm * a.ngroups;
     if (tiled_grid(a) > INT32_MAX)
         return fail(LGX_OUT_OF_BOUNDS, "tiled product of %lld workgroups", (long long)wgs);

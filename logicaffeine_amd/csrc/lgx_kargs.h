@@ -371,6 +371,7 @@ typedef struct {
     int32_t ntn, ntm;      // workgroup tiles along n and m
     int32_t grp;           // ranges per group: 1, 2 or 4 (ngroups = ceil(nranges / grp))
     int32_t swiglu;        // I of a fused SwiGLU consumer, else 0
+    int32_t whole;         // an XCD takes a run of all groups' tiles, not a share of each group's
 } lgx_gemm_tiled_args;
 
 // Grouped M > 1 products (lgx_q8_gemm_quantize_group): up to

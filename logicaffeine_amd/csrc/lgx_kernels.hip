@@ -4221,7 +4221,7 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_dequant_f16(const lgx_de
 // read into registers before the next stage's loads are issued (the
 // compiler would otherwise wait for those loads before the reads).
 // Workgroup order: physical ids go round-robin over the 8 XCDs; each XCD
-// takes a contiguous run of every group's tiles, which walk bands of 8
+// takes a contiguous run of tiles (tiled_coords), which walk bands of 8
 // activation tiles, n-tile by n-tile (activation tile fastest), so the tiles
 // in flight on one XCD share their operands through its L2.
 // ---------------------------------------------------------------------------
@@ -4235,19 +4235,25 @@ struct TgSmem {
     uint32_t dx[S][32];
 };
 
-// Group and tile of workgroup P: XCD P & 7 takes, of every group, a
-// contiguous run of ceil(tiles / 8) or one less (the runs shifted by one XCD
-// per group), so that each XCD has the same share of the last group, whose
-// ranges may be fewer (whole runs of groups per XCD: 8% more on the longest
-// one for 18944 columns); tiles walk bands of 8 activation tiles, n tile by n
-// tile.  False: no tile (the grid is padded to whole eights).
+// Group and tile of workgroup P: XCD P & 7 takes a contiguous run of ceil(T /
+// 8) tiles or one less, of all groups' tiles one after the other (a.whole: the
+// activations of a group are read by few XCDs) or of every group's (the runs
+// shifted by one XCD per group, so that each has the same share of the last
+// group, whose ranges may be fewer: whole runs take 8% longer for 18944
+// columns); tiles walk bands of 8 activation tiles, n tile by n tile.  False:
+// no tile (the grid is padded to whole eights).
 __device__ __forceinline__ bool tiled_coords(const lgx_gemm_tiled_args& a, int P, int& g, int& tn, int& tm) {
-    const int per_g = a.ntn * a.ntm, tq = (per_g + 7) >> 3, q8 = per_g >> 3, r8 = per_g & 7;
+    const int per_g = a.ntn * a.ntm, T = a.whole ? per_g * a.ngroups : per_g;
+    const int tq = (T + 7) >> 3, q8 = T >> 3, r8 = T & 7;
     const int slot = P >> 3;
     g = slot / tq;
     const int x = ((P & 7) + g) & 7, lt = slot - g * tq;
     if (lt >= q8 + (x < r8 ? 1 : 0)) return false;
-    const int rem = x * q8 + min(x, r8) + lt;
+    int rem = x * q8 + min(x, r8) + lt;
+    if (a.whole) {
+        g = rem / per_g;
+        rem -= g * per_g;
+    }
     const int band = rem / (8 * a.ntn);
     const int bsz = min(8, a.ntm - 8 * band);
     const int loc = rem - band * 8 * a.ntn;

@@ -337,6 +337,25 @@ def test_tiled64_gemm_edges_bit_exact(orc, n, k, m):
             c.close()
 
 
+@pytest.mark.parametrize("rows", [32, 64])
+@pytest.mark.parametrize("n,k,m", [(2064, 5120, 130), (208, 4160, 100), (1552, 8960, 33), (1040, 4160, 300)])
+def test_tiled_gemm_tile_orders_bit_exact(orc, n, k, m, rows):
+    """Both orders of the tiles over the XCDs, grids that are no multiple of
+    8: runs of all groups' tiles (no range missing in the last group; at most
+    one workgroup per compute unit; little missing from a small grid) and
+    shares of every group's."""
+    qs, d = orc.gen_q8_matrix(10, n + k, n, k)
+    xq, xd = orc.quantize_q8_0(orc.gen_normal_f32(10, m, (m, k)))
+    ref = orc.q8_gemm(qs, d, xq, xd)
+    for grp in (1, 2):
+        c = _ctx_with_env(LGX_GEMM_TILED_MIN=2, LGX_GEMM_TILED_ROWS=rows, LGX_GEMM_TILED_GRP=grp)
+        try:
+            y = c.q8_gemm(c.q8_matrix(qs, d), c.to_device(xq), c.to_device(xd))
+            assert np.array_equal(bits(host(y)), bits(ref)), grp
+        finally:
+            c.close()
+
+
 @pytest.mark.parametrize("n,k", [(3584, 3584), (1024, 896), (512, 2112), (64, 192), (2048, 18944)])
 @pytest.mark.parametrize("rows", [32, 64])
 def test_tiled_gemm_stage_sizes_agree(orc, n, k, rows):
