@@ -670,15 +670,18 @@ inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
 // from about 1150 (17920 x 1536 at 192 rows, 840: 37.7 against 32.1; 37888 x
 // 3584 at 100 rows, 1184: 75.0 against 84.8).  Long reductions, split into
 // several groups, gain from about 200 workgroups (1536 x 8960 at 192 rows
-// 23.4 against 25.1, 3584 x 18944 at 100 43.1 against 50.5), not at 64 rows
-// and below (35.9 against 35.3).  LGX_GEMM_TILED_ROWS forces one.
+// 23.4 against 25.1, 3584 x 18944 at 100 43.1 against 50.5).  Not at 96 rows
+// and below, where half of every second 64-row tile is empty: 37888 x 3584 at
+// 80 rows 61.8 against 55.1, 151936 x 896 60.5 against 58.3 (at 33 to 64 rows
+// 0.85-0.90 for the latter, but 1.05 and more for the others).
+// LGX_GEMM_TILED_ROWS forces one.
 inline int64_t tiled64_wgs(int n, int k, int m) {
     return (int64_t)cdiv(n, LGX_TG_N) * cdiv(m, 64) * tiled_groups(k);
 }
 inline Kern tiled_kernel(const lgx_ctx* c, int n, int k, int m) {
     if (c->tiled_rows) return c->tiled_rows >= 64 ? K_GEMM_TILED64 : K_GEMM_TILED32;
     const int64_t wgs = tiled64_wgs(n, k, m);
-    const bool wide = m > 64 && (tiled_groups(k) > 1 ? wgs >= 200 : wgs >= (m >= 256 ? 600 : 1150));
+    const bool wide = m > 96 && (tiled_groups(k) > 1 ? wgs >= 200 : wgs >= (m >= 256 ? 600 : 1150));
     return wide ? K_GEMM_TILED64 : K_GEMM_TILED32;
 }
 // Ranges per group for a product of n outputs, reduction k, over m rows

@@ -124,3 +124,11 @@ def test_products_of_the_most_rows_are_launched_whole(host, n, k, m):
         assert st == "LGX_OK"
         tiles = sum(gx for name, gx, *_ in launches if "gemm_tiled64" in name)
         assert -(-n // 64) * -(-m // 64) <= tiles < -(-n // 64) * (-(-m // 64) + 2) + 16
+
+
+@pytest.mark.parametrize("n,k", [(37888, 3584), (151936, 896), (3584, 18944), (512, 32768)])
+def test_rows_65_to_96_are_not_padded_to_128(host, n, k):
+    """Three 32-row tiles of a product, not two of 64 with the last half empty."""
+    for m, (st, launches, _) in zip(range(65, 97), host([gemm("lgx_q8_gemm", n, k, m) for m in range(65, 97)])):
+        names = [name for name, *_ in launches if "gemm_tiled" in name]
+        assert st == "LGX_OK" and len(names) == 1 and names[0].startswith("lgx_k_q8_gemm_tiled32"), (m, names)
