@@ -1629,15 +1629,17 @@ __device__ __forceinline__ void attn_stage_v(const lgx_attn_args& a, int g, int 
     }
 }
 
-// Which chains run on the matrix instruction (4 heads a step).  Measured at 32
-// sequences of 2048 tokens, 4 KV heads (VALU forms / these, us): scores and PV
-// at D = 128: 28.7 / 30.2 with one head per group, 31.8 / 31.0 with two,
-// 35.1 / 32.0 four, 43.6 / 35.8 seven, 48.7 / 36.8 eight.  At D = 64 scores
-// only (PV there has work for two waves of a single dependent chain each):
-// 16.9 / 17.8 with one head, 18.1 / 18.1 two, 20.8 / 19.3 four, 25.2 / 22.5
-// seven, 28.2 / 24.7 eight; PV too 24.8 and 26.2 with seven and eight.
-constexpr bool attn_mfma_scores(int d, int gq) { return gq >= (d == 128 ? 2 : 3); }
-constexpr bool attn_mfma_pv(int d, int gq) { return d == 128 && gq >= 2; }
+// Which chains run on the matrix instruction (4 heads a step).  D = 128, 4 KV
+// heads, 32 sequences of up to 2048 tokens, and one of 100 tokens (VALU forms /
+// scores / scores and PV, us): 23.9 / 23.5 / 26.3 and 9.4 / 9.9 / 10.3 with two
+// heads per group, 25.9 / 24.2 / 26.7 and 10.2 / 9.9 / 10.3 three; 32
+// sequences of 2048 (VALU / both) 35.1 / 32.0 four, 43.6 / 35.8 seven, 48.7 /
+// 36.8 eight.  At D = 64 scores only (PV there has work for two waves of a
+// single dependent chain each): 16.9 / 17.8 with one head, 18.1 / 18.1 two,
+// 20.8 / 19.3 four, 25.2 / 22.5 seven, 28.2 / 24.7 eight; PV too 24.8 and 26.2
+// with seven and eight.
+constexpr bool attn_mfma_scores(int, int gq) { return gq >= 3; }
+constexpr bool attn_mfma_pv(int d, int gq) { return d == 128 && gq >= 4; }
 
 template <int D, int GQ>
 __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
