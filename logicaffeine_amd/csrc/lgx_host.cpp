@@ -228,7 +228,7 @@ lgx_status lgx_quantize_q8_0(lgx_ctx* c, const float* x, int32_t m, int32_t k, i
             return fail(LGX_INVALID_ARGUMENT, "shape [%d x %d]: need m > 0, k %% 32 == 0", m, k);
         lgx_quant_args a{x, qs, d, m, k};
         return launch(c, K_QUANT,
-                      dim3((unsigned)std::min<int64_t>(((int64_t)m * (k / 4) + 255) / 256, LGX_QUANT_WGS)),
+                      dim3((unsigned)std::min<int64_t>(((int64_t)m * (k / 8) + 255) / 256, LGX_QUANT_WGS)),
                       dim3(256), a, stream);
     });
 }

@@ -30,9 +30,10 @@ typedef struct {
     uint16_t* d;      // [m][k/32]
     int32_t m, k;
 } lgx_quant_args;
-// Workgroups of a quantisation's grid at most: 2^26 threads, so that no size
-// passes the 2^32 threads of a launch; the chip holds 2048 of them at a time.
-#define LGX_QUANT_WGS (1 << 18)
+// Workgroups of a quantisation's grid at most: 2^25 threads of 8 values, so
+// that no size passes the 2^32 threads of a launch; the chip holds 2048 of them
+// at a time.
+#define LGX_QUANT_WGS (1 << 17)
 
 // One wave per (row tile of 16, range of 32 blocks[, m-group of 64 rows]).
 typedef struct {

@@ -160,22 +160,27 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_repack_t16(const lgx_rep
 }
 
 // ---------------------------------------------------------------------------
-// Q8_0 activation quantisation, eight lanes per 32-block (quantize4):
+// Q8_0 activation quantisation, four lanes per 32-block:
 //   amax = max|x|, d = amax/127, id = d ? 1/d : 0, q = clamp(round(x*id)),
 //   stored scale f16(d) (RNE).
-// Coalesced, and eight times the waves of one thread per block: 64 x 3584 with
-// the product after it 57.9 against 59.2 us; 2047 x 18944 (194 MB) 37.6
-// against 38.8.
+// Bound by memory, and by the divisions for rows of some MB: eight lanes per
+// block, which divide twice as often, took 30.1 us for 2047 x 18944 (194 MB) and
+// 6.8 for 2047 x 3584, this 27.6 and 5.9; one thread per block (uncoalesced, an
+// eighth of the waves) 28.9 and 7.7, and 4.0 against 3.2 for 64 x 18944.
 // ---------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(256) void lgx_k_quantize_q8_0(const lgx_quant_args a) {
-    const int64_t n = (int64_t)a.m * (a.k >> 2);   // four values each
-    // The grid is capped (LGX_QUANT_WGS); whole 8-lane groups end together.
+    const int64_t n = (int64_t)a.m * (a.k >> 3);   // eight values each
+    // The grid is capped (LGX_QUANT_WGS); whole 4-lane groups end together.
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const float4 v = ((const float4*)a.x)[i];
-        const float f[4] = {v.x, v.y, v.z, v.w};
+        const float4 v = ((const float4*)a.x)[2 * i], w = ((const float4*)a.x)[2 * i + 1];
+        const float f[4] = {v.x, v.y, v.z, v.w}, g[4] = {w.x, w.y, w.z, w.w};
+        float am = fmaxf(absmax4(f), absmax4(g));
+        am = fmaxf(am, dpp_f<0xB1>(am));
+        am = fmaxf(am, dpp_f<0x4E>(am));
         uint16_t dh;
-        ((uint32_t*)a.qs)[i] = quantize4(f, dh);
-        if ((threadIdx.x & 7) == 0) a.d[i >> 3] = dh;
+        const uint32_t q0 = quantize4_am(f, am, dh), q1 = quantize4_am(g, am, dh);
+        ((uint2*)a.qs)[i] = make_uint2(q0, q1);
+        if ((threadIdx.x & 3) == 0) a.d[i >> 2] = dh;
     }
 }
 

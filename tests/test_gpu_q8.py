@@ -59,7 +59,7 @@ def test_quantize_bit_exact(ctx, orc, m, k):
 
 
 def test_quantize_more_values_than_one_pass_of_the_grid(ctx, orc):
-    """2^18 workgroups take 2^28 values a pass: the rows on both sides of the
+    """2^17 workgroups take 2^28 values a pass: the rows on both sides of the
     first pass's end, and the last, against the oracle."""
     m, k = 8195, 32768
     x = ctx.torch.zeros(m, k, dtype=ctx.torch.float32, device=ctx.dev)
