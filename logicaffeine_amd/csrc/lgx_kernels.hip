@@ -1733,13 +1733,14 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
 #pragma unroll
         for (int j = 0; j < CPR; ++j) kv[j] = kr[j];
     }
-    // D = 128: the K row has arrived before V is requested (once direct loads
-    // are in flight the compiler waits for every load before the first use of
-    // any), so V's transfer overlaps the score chain: 79.2 against 79.9 us for
-    // 64 sequences of up to 4096 tokens.  D = 64, whose grids leave memory idle
-    // at the start, requests both at once (17.2 against 17.7 us for 32
-    // sequences of 2048).
-    if constexpr (D == 128) {
+    // The K row has arrived before V is requested (once direct loads are in
+    // flight the compiler waits for every load before the first use of any), so
+    // V's transfer overlaps the score chain: 79.2 against 79.9 us for 64
+    // sequences of up to 4096 tokens (D = 128), 23.4 against 24.1 for 64 of up to
+    // 1024, 16/8 heads of 64.  D = 64 with matrix scores, whose short chain would
+    // not cover it, requests both at once and waits once, ahead of the scores
+    // (17.2 against 17.7 us for 32 sequences of 2048).
+    if constexpr (D == 128 || !MS) {
 #pragma unroll
         for (int j = 0; j < CPR; ++j)
             asm volatile("" : "+v"(kv[j].x), "+v"(kv[j].y), "+v"(kv[j].z), "+v"(kv[j].w));
