@@ -596,11 +596,11 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
         // the tiled product from 17 rows (config 1 at M = 32: 28.9 us against
         // 35.4 us per step on the 16-row streaming kernels)
         const bool tiled = m >= std::min(c->tiled_min, 17);
-        // 64-row tiles where they are worth it for the grid of all matrices
+        // 64-row tiles where the grid of all matrices fills the device
         int64_t wgs64 = 0;
         for (int i = 0; i < count; ++i) wgs64 += tiled64_wgs(W[i].n, W[i].k, m);
         const Kern tk = c->tiled_rows ? tiled_kernel(c, W[0].n, W[0].k, m)
-                        : m >= 256 && wgs64 >= 600 ? K_GEMM_TILED64 : K_GEMM_TILED32;
+                        : tiled64_fills(wgs64, m) ? K_GEMM_TILED64 : K_GEMM_TILED32;
         const int trows = tiled_rows_of(tk);
         // ranges per group of the tiled products: 2, or 1 when that leaves
         // fewer than two workgroups per compute unit over all the matrices

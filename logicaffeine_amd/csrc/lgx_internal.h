@@ -678,10 +678,19 @@ inline lgx_status run_q8_tiled(lgx_ctx* c, const lgx_q8_matrix* W, const int8_t*
 inline int64_t tiled64_wgs(int n, int k, int m) {
     return (int64_t)cdiv(n, LGX_TG_N) * cdiv(m, 64) * tiled_groups(k);
 }
+// Whether a grid of wgs 64-row workgroups fills the device, for a product in
+// one group or several matrices in one launch.  Grouped calls, whose ranges go
+// in groups of 1 or 2 (64 against 32 rows, us): 37888 x 3584 at 100 / 192 /
+// 255 rows 77 against 94, 116 against 135, 152 against 176 (at 80 rows 74
+// against 70); its MLP with 3584 x 18944 at 100 / 255 119 against 141, 239
+// against 273; below the line the MLP of 1536 x 8960 at 129 / 160 rows (1056
+// workgroups) 44.0 against 42.9 and 45.0 against 43.9, of 896 x 4864 at 129 /
+// 224 (540, 720) 27.8 against 25.1 and 32.4 against 29.8.
+inline bool tiled64_fills(int64_t wgs, int m) { return m > 96 && wgs >= (m >= 256 ? 600 : 1150); }
 inline Kern tiled_kernel(const lgx_ctx* c, int n, int k, int m) {
     if (c->tiled_rows) return c->tiled_rows >= 64 ? K_GEMM_TILED64 : K_GEMM_TILED32;
     const int64_t wgs = tiled64_wgs(n, k, m);
-    const bool wide = m > 96 && (tiled_groups(k) > 1 ? wgs >= 200 : wgs >= (m >= 256 ? 600 : 1150));
+    const bool wide = tiled64_fills(wgs, m) || (m > 96 && tiled_groups(k) > 1 && wgs >= 200);
     return wide ? K_GEMM_TILED64 : K_GEMM_TILED32;
 }
 // Ranges per group for a product of n outputs, reduction k, over m rows

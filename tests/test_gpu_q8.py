@@ -294,10 +294,10 @@ def test_special_scales_bit_exact(ctx, orc, m, tiled_rows):
     assert np.array_equal(y, ref, equal_nan=True)
 
 
-@pytest.mark.parametrize("rows,grp", [(128, 0), (64, 0), (32, 0), (64, 1), (64, 2), (32, 4), (128, 1)])
+@pytest.mark.parametrize("rows,grp", [(64, 0), (32, 0), (64, 1), (32, 1), (64, 2), (32, 4), (64, 4)])
 def test_tiled_gemm_small_m_forced(ctx, orc, rows, grp):
     """LGX_GEMM_TILED_MIN=2 routes every m > 1 through the tiled product with
-    128, 64 or 32 activation rows per workgroup and 1, 2 or 4 ranges per
+    64 or 32 activation rows per workgroup and 1, 2 or 4 ranges per
     group (0: chosen by grid size): a ragged row tile, rows spanning
     workgroup tiles and 9 ranges (groups of 4 + 4 + 1, 2 + 2 + 2 + 2 + 1, or
     single ranges) agree with the oracle."""
@@ -357,12 +357,11 @@ def test_tiled_gemm_tile_orders_bit_exact(orc, n, k, m, rows):
 
 
 @pytest.mark.parametrize("n,k", [(3584, 3584), (1024, 896), (512, 2112), (64, 192), (2048, 18944)])
-@pytest.mark.parametrize("rows", [32, 64])
+@pytest.mark.parametrize("rows", [32])
 def test_tiled_gemm_stage_sizes_agree(orc, n, k, rows):
-    """Grids of at most two workgroups per compute unit run in stages of 4
-    pairs, larger ones in stages of 2 (LGX_TILED_S4=0: always 2).  Both
-    stage sizes give the oracle's bits at 32 and 64 activation rows per
-    workgroup: whole ranges (3584), a range of 14 pairs ending mid-stage
+    """32-row grids of at most two workgroups per compute unit run in stages
+    of 4 pairs, larger ones in stages of 2 (LGX_TILED_S4=0: always 2).  Both
+    stage sizes give the oracle's bits: whole ranges (3584), a range of 14 pairs ending mid-stage
     (896), 33 pairs (2112), 3 pairs (192) and 19 ranges in groups (18944)."""
     qs, d = orc.gen_q8_matrix(5, n + k, n, k)
     x = orc.gen_normal_f32(5, rows, (64, k))
@@ -562,11 +561,13 @@ def test_grouped_gemm_small_m_one_launch(ctx, orc, m):
     c3.close()
 
 
-@pytest.mark.parametrize("m,env", [(160, {}), (64, dict(LGX_GEMM_TILED_ROWS="64"))],
-                         ids=["tiled128-rows", "tiled64-rows"])
-def test_grouped_gemm_other_kernel_forms(orc, m, env):
-    """The grouped product's other tiled forms: 128-row tiles (m >= 128) and
-    64-row tiles (forced), each output bit-identical to the oracle."""
+@pytest.mark.parametrize("m,env,kernel", [(160, {}, "tiled32"), (257, {}, "tiled64"), (520, {}, "tiled64"),
+                                          (64, dict(LGX_GEMM_TILED_ROWS="64"), "tiled64")])
+def test_grouped_gemm_other_kernel_forms(orc, m, env, kernel):
+    """The grouped product's tiled forms by its own rule and forced: 32-row
+    tiles below the grid that fills the device, 64-row tiles from it on (five
+    and nine tiles along m, bands of eight), each output bit-identical to the
+    oracle."""
     c = _ctx_with_env(**env)
     shapes = [(8960, 1536), (1536, 8960), (80, 1088)]
     Ws, xs, refs = [], [], []
@@ -577,9 +578,11 @@ def test_grouped_gemm_other_kernel_forms(orc, m, env):
         Ws.append(c.q8_matrix(qs, d))
         xs.append(c.to_device(x))
         refs.append(orc.q8_gemm(qs, d, xq, xd))
+    c.kernel_timing(True)
     ys = c.q8_gemm_quantize_group(Ws, xs)
     for i, (y, ref) in enumerate(zip(ys, refs)):
         assert np.array_equal(bits(host(y)), bits(ref)), (m, shapes[i])
+    assert c.kernel_stats(f"lgx_k_q8_gemm_{kernel}_group")[0] == 1
     del Ws, xs, ys
     c.close()
 

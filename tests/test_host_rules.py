@@ -132,3 +132,19 @@ def test_rows_65_to_96_are_not_padded_to_128(host, n, k):
     for m, (st, launches, _) in zip(range(65, 97), host([gemm("lgx_q8_gemm", n, k, m) for m in range(65, 97)])):
         names = [name for name, *_ in launches if "gemm_tiled" in name]
         assert st == "LGX_OK" and len(names) == 1 and names[0].startswith("lgx_k_q8_gemm_tiled32"), (m, names)
+
+
+@pytest.mark.parametrize("shapes,ms,rows", [
+    ([(37888, 3584)], range(97, 256, 6), 64), ([(37888, 3584)], range(17, 97, 5), 32),
+    ([(18944, 3584)] * 2 + [(3584, 18944)], range(97, 300, 9), 64), ([(8960, 1536)] * 2, range(97, 193, 9), 32),
+    ([(4864, 896), (896, 4864)], [100, 160, 255], 32), ([(8960, 1536)], [257, 520], 64)])
+def test_grouped_products_take_the_row_tile_of_their_whole_grid(host, shapes, ms, rows):
+    """One rule for a product in one group and for several matrices in one
+    launch (37888 x 3584 alone and grouped took different tiles at 97..255
+    rows)."""
+    def group(m):
+        return ["lgx_q8_gemm_quantize_group", [len(shapes), [dict(n=n, k=k) for n, k in shapes], [PTR] * len(shapes), m,
+                                               [PTR] * len(shapes), None]]
+    for m, (st, launches, _) in zip(ms, host([group(m) for m in ms])):
+        names = [name for name, *_ in launches if "gemm_tiled" in name]
+        assert st == "LGX_OK" and names == [f"lgx_k_q8_gemm_tiled{rows}_group"], (m, names)
