@@ -244,6 +244,76 @@ def test_prefill_attn_more_chunks_than_a_grid_dimension(ctx, orc):
     assert np.array_equal(out, prefill_ref(orc, q, k, v, pt, [ctx_len], P))
 
 
+def extreme_inputs(orc, hq, hkv, d, lens, rows, seed):
+    """Cache and query rows that reach every part of binary32 in the two
+    chains: binary16-subnormal K and V values and zeros among normal ones,
+    query rows so small that products are subnormal or vanish, one large row
+    whose scores lie from just below the -87.33 cutoff up to 0 (the
+    probabilities near 2^-126 times subnormal V), an infinite and a NaN row."""
+    k, v, pt, _ = make_cache(len(lens), hkv, d, lens, seed)
+    rng = np.random.default_rng(seed)
+    for a in (k, v):
+        m = rng.random(a.shape)
+        a[m < 0.3] &= 0x83ff                             # subnormal, both signs
+        a[m < 0.1] &= 0x8000                             # zeros
+    q = orc.gen_normal_f32(8, seed, (rows, hq, d))
+    scale = np.float32([1.0, 1e-38, 1e-40, 1e-33])
+    q *= scale[rng.integers(0, 4, (rows, hq, 1))]
+    # dimension 0 alone decides the scores of these rows: 0 at the first cached
+    # token, whose V is 0, and -86.9 to -87.4 elsewhere
+    q[1::5] = 0.0
+    q[1::5, :, 0] = np.sqrt(d) / 8
+    for b, n in enumerate(lens):
+        k0 = -(np.float32(695.0) + 4 * rng.random((n, hkv), dtype=np.float32))
+        for t in range(n):
+            k[pt[b, t // 16], :, t % 16, 0] = k0[t].astype(np.float16).view(np.uint16)
+        k[pt[b, 0], :, 0, 0] = 0
+        v[pt[b, 0], :, 0] = 0
+    q[3, 0, 1] = np.inf
+    q[3, -1, 2] = np.nan
+    return q, k, v, pt
+
+
+def assert_bits(out, ref):
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(out), nan)
+    assert np.array_equal(out.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(2, 2, 64), (8, 2, 64), (7, 1, 64), (16, 2, 64), (2, 2, 128), (3, 1, 128),
+                                      (8, 2, 128), (7, 1, 128), (8, 1, 128)])
+def test_decode_attn_subnormal_infinite_and_nan_operands(ctx, orc, hq, hkv, d):
+    """The matrix-instruction chains (and the fmaf forms of few heads) round
+    every step like fmaf also where operands, products or sums are subnormal,
+    infinite or NaN: chunk tails of 1 to 15 tokens, one and two V stages."""
+    lens = [1, 7, 31, 128, 143, 255, 300, 529, 64, 17]
+    q, k, v, pt = extreme_inputs(orc, hq, hkv, d, lens, len(lens), seed=hq + d)
+    ref = orc.gqa_decode_attn(q, k, v, pt, np.asarray(lens, np.int32))
+    fin = np.abs(ref[np.isfinite(ref)])
+    assert ((fin > 0) & (fin < 1.17e-38)).any() and np.isnan(ref[3]).any()
+    assert_bits(run(ctx, q, k, v, pt, lens), ref)
+
+
+@pytest.mark.parametrize("rows", [16, 32])
+@pytest.mark.parametrize("hq,hkv,d,P", [(2, 2, 64, 40), (7, 1, 64, 9), (8, 1, 128, 9), (2, 2, 128, 35), (6, 2, 128, 21)])
+def test_prefill_attn_subnormal_infinite_and_nan_operands(monkeypatch, orc, rows, hq, hkv, d, P):
+    """The same through both block sizes of the exact prefill attention, whose
+    last token groups hold rows of different lengths."""
+    monkeypatch.setenv("LGX_PFA_ROWS", str(rows))
+    ctx_len = [0, 250, 19]
+    lens = [n + P for n in ctx_len]
+    q, k, v, pt = extreme_inputs(orc, hq, hkv, d, lens, 3 * P, seed=hq + d + P)
+    ref = prefill_ref(orc, q, k, v, pt, ctx_len, P)
+    fin = np.abs(ref[np.isfinite(ref)])
+    assert ((fin > 0) & (fin < 1.17e-38)).any() and np.isnan(ref[3]).any()
+    c = lgx.Context(0)
+    try:
+        assert_bits(host(c.gqa_prefill_attn(c.to_device(q), c.to_device(k), c.to_device(v), c.to_device(pt),
+                                            c.to_device(np.asarray(ctx_len, np.int32)), P, max(lens))), ref)
+    finally:
+        c.close()
+
+
 def test_prefill_attn_config4_shape_sampled(ctx, orc):
     """Config-4 head layout at a 4096-token context: 64 new rows after 4032
     cached tokens (17 chunks), checked on a sample of rows."""

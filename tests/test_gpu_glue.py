@@ -165,7 +165,7 @@ def test_lm_head_f16_bit_exact(ctx, orc, m, h, vocab):
                                        (64, 1024, 4160), (32, 896, 151936), (5, 1536, 1000),
                                        (20, 3072, 700), (2, 8192, 130)])
 def test_lm_head_f16_t64_bit_exact(ctx, orc, m, h, vocab):
-    """The T64 path (repacked embedding, activations in SGPRs) gives the
+    """The T64 path (repacked embedding, activations in T16 columns) gives the
     oracle's logits bit for bit, including a ragged last row group and a
     partial last group of 16 activation rows."""
     rng = np.random.default_rng(m + h + vocab)
@@ -184,6 +184,33 @@ def test_lm_head_f16_t64_bit_exact(ctx, orc, m, h, vocab):
         assert np.array_equal(bits(out[:, rows]), bits(orc.lm_head_f16(x, E[rows])))
     else:
         assert np.array_equal(bits(out), bits(orc.lm_head_f16(x, E)))
+
+
+@pytest.mark.parametrize("m,h,vocab", [(18, 256, 330), (5, 1536, 200)])
+def test_lm_head_f16_t64_subnormal_infinite_and_nan_operands(ctx, orc, m, h, vocab):
+    """Each step of the matrix-instruction chains rounds like fmaf where
+    activations, embedding entries, products or sums are subnormal, infinite
+    or NaN."""
+    rng = np.random.default_rng(m + h)
+    x = rng.standard_normal((m, h)).astype(np.float32)
+    x *= np.float32([1.0, 1e-38, 1e-40, 1e-33, 1e-44])[np.arange(m) % 5][:, None]
+    x[0] = np.where(rng.random(h) < 0.5, x[0], x[0] * np.float32(1e-39))
+    x[0, h - 16:] = np.float32(1e-42)
+    E = orc.f32_to_f16((rng.standard_normal((vocab, h)) * 0.02).astype(np.float32))
+    sub = rng.random(E.shape)
+    E[sub < 0.5] &= 0x83ff
+    E[sub < 0.1] &= 0x8000
+    E[3] &= 0x83ff                               # a row of subnormals only
+    x[m - 1, 5] = np.inf
+    x[m - 2, h - 1] = np.nan
+    E[7, 9] = 0x7c00
+    out = host(ctx.lm_head_f16_t64(ctx.to_device(x), ctx.f16_repack_t64(ctx.to_device(E)), vocab))
+    ref = orc.lm_head_f16(x, E)
+    nan = np.isnan(ref)
+    fin = np.abs(ref[np.isfinite(ref)])
+    assert ((fin > 0) & (fin < 1.17e-38)).any() and nan.any() and np.isinf(ref).any()
+    assert np.array_equal(np.isnan(out), nan)
+    assert np.array_equal(bits(out)[~nan], bits(ref)[~nan])
 
 
 def test_lm_head_one_hot_selects_embedding_column(ctx, orc):
