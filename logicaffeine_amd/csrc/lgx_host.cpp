@@ -400,6 +400,7 @@ lgx_status lgx_gqa_decode_attn(lgx_ctx* c, const float* q, const uint16_t* kpage
         a.scale = (float)(1.0 / std::sqrt((double)d));
         st = ensure_ws(c, (size_t)B * hq * a.nchunk * (d + 2) * sizeof(float), &a.part);
         if (st != LGX_OK) return st;
+        a.rot = attn_rot(a.nchunk);
         st = launch(c, (Kern)k, dim3(a.nchunk, B * hkv), dim3(256), a, stream);
         if (st != LGX_OK) return st;
         return launch(c, d == 64 ? K_ATTN_COMBINE_D64 : K_ATTN_COMBINE_D128, dim3(B * hq), dim3(d),

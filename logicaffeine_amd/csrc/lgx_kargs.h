@@ -107,6 +107,7 @@ typedef struct {
     int32_t qpr;
     int32_t ncg;               // prefill: chunks covered by the grid
     int32_t pfa_fold;          // prefill: chunks along x (set by the launch)
+    uint32_t rot;              // decode: attn_rot(nchunk)
     int32_t xq_t16;            // combine+quantise: xq in T16 tiles instead of row-major
     uint16_t* out16;           // fast prefill attention: binary16 out rows [rows][hq*d] (nullable)
 } lgx_attn_args;

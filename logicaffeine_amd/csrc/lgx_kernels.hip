@@ -1665,17 +1665,8 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     __shared__ int pg_s[C / LGX_PAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // with a multiple of 8 chunks per row, workgroup x of a row takes chunk (x +
-    // row) mod nchunk: ids go round-robin over the 8 XCDs, and an XCD would
-    // otherwise hold the same chunk index of every sequence (few of which reach
-    // the late chunks).  Other counts space the live chunks evenly as they are:
-    // rotated, two of them meet on some compute units while others have none
-    // (32 sequences of 144 tokens, 3 chunks, 28/4 heads of 128: 17.7 against 13.2
-    // us; 16 of 900, 12 chunks, 25.3 against 15.6; the other way round 64 of 130,
-    // 12 chunks, 24.8 against 30.2).  672 mixes of 2 to 12 chunks: 0.90 of the
-    // time before the rotation, at most 1.04; all rotated 0.92 and 1.34
-    const int bg = blockIdx.y;
-    const int c = gridDim.x & 7 ? (int)blockIdx.x : (int)((blockIdx.x + blockIdx.y) % gridDim.x);
+    // attn_rot's rotation of the chunks by the row
+    const int bg = blockIdx.y, c = (blockIdx.x & ~a.rot) | ((blockIdx.x + bg) & a.rot);
     const int b = bg / a.hkv, g = bg - b * a.hkv;
     const int h0 = g * GQ;
     // the query rows as the matrix A operand, requested first: lane l of

@@ -514,6 +514,7 @@ lgx_status layers(lgx_model* md, int B, const int32_t* tokens, int tokens_stride
         aa.hkv = hkv;
         aa.maxp = md->maxp;
         aa.nchunk = md->nchunk;
+        aa.rot = attn_rot(md->nchunk);
         aa.num_pages = md->num_pages;
         aa.maxlen = cf.max_seq;
         aa.len_add = 1;
