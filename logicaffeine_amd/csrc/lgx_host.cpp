@@ -688,6 +688,9 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
             lgx_tiled_group_args ta{};
             ta.count = count;
             ta.wg0[0] = 0;
+            int64_t wgs = 0;
+            for (int i = 0; i < count; ++i)
+                wgs += (int64_t)cdiv(W[i].n, LGX_TG_N) * cdiv(m, trows) * tiled_groups(W[i].k, grp);
             for (int i = 0; i < count; ++i) {
                 lgx_gemm_tiled_args& a = ta.mat[i];
                 a.wt = W[i].qs;
@@ -702,7 +705,7 @@ lgx_status lgx_q8_gemm_quantize_group(lgx_ctx* c, int32_t count, const lgx_q8_ma
                 a.ngroups = tiled_groups(W[i].k, grp);
                 a.ntn = (int)cdiv(W[i].n, LGX_TG_N);
                 a.ntm = (int)cdiv(m, trows);
-                a.whole = tiled_whole(c, a, trows);
+                a.whole = tiled_whole(c, a, trows, wgs);
                 const int64_t end = ta.wg0[i] + tiled_grid(a);
                 if (end > INT32_MAX) return fail(LGX_OUT_OF_BOUNDS, "grouped product too large");
                 ta.wg0[i + 1] = (int32_t)end;
