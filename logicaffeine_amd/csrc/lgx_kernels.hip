@@ -1565,8 +1565,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // loads (global_load_lds_dwordx4, 1 KiB per wave instruction) bring the
 // first 32 KiB of the chunk's V rows into LDS in token order (the whole
 // chunk at D = 64, tokens 0..127 at D = 128; at D = 128 each thread also
-// loads 128 bytes of tokens 128..255 into registers), and V lands while the
-// scores are computed.  Phase 1: thread t's token's canonical score chain
+// loads 128 bytes of tokens 128..255 into registers).  V lands while the
+// scores are computed, but at D = 64 with matrix scores, which wait for K and V
+// together.  Phase 1: thread t's token's canonical score chain
 // over d for the GQ heads.  Phase 2: per head the chunk max (exact in any
 // order), p_t = lgx_expf(s_t - m), and the halving-tree sum of the 256 slots.
 // Phase 3: the canonical chain over the chunk's tokens, o[i] = fmaf(p_t,
@@ -1698,7 +1699,8 @@ __device__ __forceinline__ void attn_chunk_body(const lgx_attn_args& a) {
     const int n = min(C, L - t0);
     // D = 64: every thread looks up its own token's page, so no LDS round and
     // no barrier stand before the K loads; D = 128 shares the chunk's 16
-    // entries in LDS.  The entries were requested with the length; a token
+    // entries in LDS.  (The compiler issues the entries' load behind the exit
+    // above, i.e. after the length.)  A token
     // past the end reads a real slot that the wave (D = 64: lane 0's) or the
     // pool (D = 128: page 0) has anyway, never used.
     const bool valid = tid < n;
@@ -4097,7 +4099,7 @@ extern "C" __global__ __launch_bounds__(64) void lgx_k_sample_final(const lgx_sa
     const uint64_t* lists = a.cand + (int64_t)b * a.nslices * LGX_SAMPLE_MAX_K;
     const int pos = a.pos ? a.pos[b] : a.seq_len[b];
     // list s at ls + s * (top_k + 1): the heads of the lanes' lists spread
-    // over the banks, an empty key behind each list
+    // over the banks
     const int ld = a.top_k + 1;
     for (int i = l; i < a.nslices * a.top_k; i += 64) {
         const int s = i / a.top_k, r = i - s * a.top_k;
@@ -4489,7 +4491,7 @@ __device__ __forceinline__ void q8_tiled_body(const lgx_gemm_tiled_args& a, cons
 // v_mfma_i32_32x32x32_i8 is one block's dots of 1024 outputs and one rank-1
 // v_mfma_f32_32x32x8_f16 their scale products, half the matrix cycles per
 // output of the 16 x 16 forms (9.1 + 8.4 against 17.4 + 17.3 per 256
-// outputs), which leaves the epilogue's convert and fma (VALU, 79% busy) as the
+// outputs), which leaves the epilogue's convert and fma (VALU, 88% busy) as the
 // bound.  Wave (wn, wm) owns weight rows 32 wn .. + 31 against activation
 // rows 32 wm .. + 31; lane l = row + 32 h of an operand reads the 8-byte
 // chunks 2h and 2h + 1 of its row and block (the same columns for both
@@ -4770,8 +4772,8 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 //            neighbours in LDS: pfa_pos), B = V through the transposing LDS
 //            load.  V passes through two 8 KiB buffers by direct
 //            global->LDS loads, 16-byte pieces swizzled by the row.
-// Memory rounds in a row, which are what a few rows' call waits for: the page
-// entry with the length; the query rows and the K row; the first two V stages
+// Memory rounds in a row, which are what a few rows' call waits for: the
+// length; the page entry; the query rows and the K row; the first two V stages
 // during the score chain; each later one during the stage before it.  (The V
 // loads stand in inline assembly: with those it knows, the compiler moved the
 // first stage behind the score chain and waited for the next stage's before
@@ -4781,8 +4783,9 @@ extern "C" __global__ __launch_bounds__(256) void lgx_k_q8_combine_group(const l
 // rows, query values through scalar registers).
 // 50 or 33 KiB of LDS and at most 168 or 128 VGPRs: three or four workgroups
 // per compute unit, whose softmax and loads overlap the others' matrix work.
-// Bound by the binary32 matrix rate (65 cycles for 2048 products; 140 us of
-// it below) and the softmax's VALU work.  8 sequences x 128 rows at contexts
+// Bound by the binary32 matrix rate (65 cycles for 2048 products) and the
+// softmax's and conversions' VALU work: the matrix units are busy for 0.53 of
+// the cycles of the call below, the VALU for 0.33.  8 sequences x 128 rows at contexts
 // up to 2000, 28/4 heads of 128, same inputs again and again: 205 us, 222
 // before the rounds above were taken out, 647 on the VALU.
 // Rows of a block end at different tokens: p is 0 past a row's length, which
@@ -4849,7 +4852,8 @@ __device__ __forceinline__ void attn_prefill_body(const lgx_attn_args& a) {
     if (qb >= nqb) return;
     const int b = bg / a.hkv, g = bg - b * a.hkv;
     const int j0 = qb * QB, t0 = c * C;
-    // the page entry of thread t's own token, requested with the length
+    // the page entry of thread t's own token (the compiler issues the load
+    // behind the exit below, i.e. after the length)
     const int pge = a.page_table[(int64_t)b * a.maxp + min((t0 + tid) / LGX_PAGE, a.maxp - 1)];
     const int sl = a.seq_len[b];
     // tokens of this chunk that query row j of the sequence attends to

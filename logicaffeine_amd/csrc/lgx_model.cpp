@@ -306,9 +306,13 @@ bool dec_tiled(const lgx_model* md, int m) { return m >= 33 && !md->ctx->decode_
 // Decode tiled kernel for W over m rows: 64 activation rows per workgroup
 // (each weight tile read by one workgroup, not two) for the products whose
 // 32-row grid holds more than four workgroups per compute unit, 32 rows for
-// the small ones (config 4, per launch: lm_head 160 against 174 us, gate|up
-// 50.4 against 51.5, down 30.6 against 31.8; qkv 13.4 against 11.9, o 10.2
-// against 8.8).  LGX_GEMM_TILED_ROWS forces one width.
+// the small ones (7B shape, 64 rows, per launch in the step: gate|up with its
+// SwiGLU 49.0 against 51.3 us, down 27.8 against 28.0, a 32000-row lm_head 41.9
+// against 42.6; qkv 11.8 against 11.3, o 10.8 against 8.8; a step of 8 layers
+// and 64 / 49 rows 1180 / 1125 us, 1184 / 1155 on 32-row tiles, 1192 / 1137 on
+// 64-row ones).  lgx_q8_gemm's rule is tiled_kernel's: it takes 32 rows up to
+// 96, where only the largest grids gain from 64.  LGX_GEMM_TILED_ROWS forces
+// one width.
 Kern dec_kernel(const lgx_model* md, const DevQ8& W, int m) {
     const lgx_ctx* c = md->ctx;
     if (c->tiled_rows || m < 49) return tiled_kernel(c, W.m.n, W.m.k, m);
