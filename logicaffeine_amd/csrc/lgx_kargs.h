@@ -350,7 +350,7 @@ typedef struct {
     float top_p, inv_temp;
 } lgx_sample_args;
 
-// Large-M Q8_0 product (prefill): one workgroup per (64 weight rows, 128
+// Large-M Q8_0 product (prefill): one workgroup per (64 weight rows, 64 or 32
 // activation rows, group of LGX_TG_RANGES ranges).  Activations in the T16
 // tile layout of the weights (row tiles of 16, 1 KiB per 64-column pair).
 // part[g][m][n] = canonical tree over the ranges of group g, so the tree
